@@ -144,6 +144,10 @@ int rk_npu_hip_inject_alloc_failures(int count);
  *                    64x128, 32x128 or 192x256 GEMM tile
  *   HM_SPLITS        0 by shape; n > 0 forces n K pieces per GEMM tile
  *   HM_FORCE_GEMM    1: rows <= 8 take the MFMA GEMM instead of the GEMV
+ *   HM_SKINNY        -1 by shape; 0 never, 1 always (up to 256 rows): the
+ *                    kernel that streams the weights into matrix-core
+ *                    operands instead of the GEMV or the tiled GEMM (not when
+ *                    HM_GEMM_VARIANT or HM_SPLITS force the latter)
  *   HM_GEMV_QW       -1 by shape; 0 never, 1 always (when the rows fit) a
  *                    quantization wave in the GEMV blocks
  *   HM_GEMV_SPLITS   0 by shape; n > 0 forces n K pieces of the one-row GEMV
@@ -196,8 +200,11 @@ int rk_npu_hip_profile_begin(int max_launches);
 int rk_npu_hip_profile_end(void);
 int rk_npu_hip_profile_read(rk_npu_hip_kernel_stat* stats, int capacity, int* count);
 
-/* Launch plan the library uses for a linear of this shape, for diagnostics:
- * kind 0 = GEMV (no MFMA), 1 = MFMA GEMM; tile sizes and K splits. */
+/* Launch plan of a linear of this shape, for diagnostics: kind 0 = GEMV, 1 =
+ * tiled MFMA GEMM; tile sizes and K splits. It is the plan that sizes the
+ * workspace and that HM_SKINNY=0 launches: by default most calls of 3 to 64
+ * rows, and of up to 256 where few column tiles share the codes, run on the
+ * streaming kernel instead (HM_SKINNY). */
 typedef struct rk_npu_hip_plan {
     int32_t kind;
     int32_t block_m;

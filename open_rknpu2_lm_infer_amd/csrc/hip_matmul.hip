@@ -306,7 +306,8 @@ static const int kBN[] = {256, 128, 128, 128, 128, 256};
 // variable, read once when the library first plans a launch; afterwards only
 // rk_npu_hip_set_switch changes it, so no launch reads the environment.
 enum SwitchId { SW_GEMM_VARIANT, SW_SPLITS, SW_FORCE_GEMM, SW_GEMV_QW, SW_GEMV_SPLITS, SW_FFN_FUSED, SW_FFN_SPIN,
-                SW_GEMV_PREQ, SW_HOST_SPIN, SW_GEMV_COMBINE, SW_HOST_FLAG, SW_HOST_POLL, SW_COUNT };
+                SW_GEMV_PREQ, SW_HOST_SPIN, SW_GEMV_COMBINE, SW_HOST_FLAG, SW_HOST_POLL, SW_SKINNY,
+                SW_COUNT };
 struct SwitchDef {
     const char* name;
     int fallback;
@@ -314,7 +315,8 @@ struct SwitchDef {
 static const SwitchDef kSwitches[SW_COUNT] = {
     {"HM_GEMM_VARIANT", -1}, {"HM_SPLITS", 0},         {"HM_FORCE_GEMM", 0}, {"HM_GEMV_QW", -1},
     {"HM_GEMV_SPLITS", 0},   {"HM_FFN_FUSED", 0},      {"HM_FFN_SPIN", 1 << 16}, {"HM_GEMV_PREQ", -1},
-    {"HM_HOST_SPIN", 0},     {"HM_GEMV_COMBINE", 1},   {"HM_HOST_FLAG", 1},       {"HM_HOST_POLL", 2000}};
+    {"HM_HOST_SPIN", 0},     {"HM_GEMV_COMBINE", 1},   {"HM_HOST_FLAG", 1},       {"HM_HOST_POLL", 2000},
+    {"HM_SKINNY", -1}};
 
 static std::atomic<int>* switch_table() {
     static std::atomic<int> table[SW_COUNT];
@@ -440,6 +442,43 @@ Plan plan_linear(int rows, const Geometry& g) {
     return plan_gemm(rows, g, -1);
 }
 
+// --- few rows: skinny_kernel ---------------------------------------------------
+constexpr int SKINNY_MAX_ROWS = 256;
+
+// Whether a call of `rows` rows runs on skinny_kernel, and how. Lines drawn by
+// measurement (per call with the quantization launch, us, other path -> this):
+// - 1 or 2 rows stay with the GEMV, which needs no quantization launch (qkv
+//   2560x6144 W4 of 2 rows 6.3 -> 7.3). 3 or 4 rows of W4 come here (gate_up
+//   2560x19456 13.4 -> 11.6, down 9728x2560 11.2 -> 10.8, qkv 8.0 -> 7.3), of
+//   W8 they stay (up 2560x9728 9.8 -> 11.1). 5 to 8 rows come here (W4 qkv
+//   9.3 -> 7.4, gate_up 16.9 -> 11.7; W8 o 9.8 -> 8.5, gate_up 19.2 -> 17.2).
+// - up to 64 rows every measured shape gains (skinny.hpp).
+// - above, up to 256, the codes a CU reads decide: blocks per CU, rounded up,
+//   times the block's rows, times K. qkv of 128 rows (320 KB) 15.2 -> 12.2 and
+//   o 4096x2560 of 128 (512 KB) 19.7 -> 13.0, of 256 (512 KB) 20.5 -> 15.0;
+//   qkv of 256 (640 KB) 16.1 -> 19.2, up 2560x9728 of 128 (640 KB) 16.4 -> 18.7.
+// - one column tile per block while the blocks fit one per CU, else two (o of
+//   16 rows W4 one 7.5, two 8.1; qkv 7.8 and 7.5, of 128 rows 14.5 and 12.2).
+// HM_SKINNY: 0 never, 1 always up to SKINNY_MAX_ROWS rows. A forced GEMM tile
+// or split (HM_GEMM_VARIANT, HM_SPLITS) keeps the tiled GEMM.
+constexpr size_t skinny_code_bytes = (size_t)576 << 10;
+
+static bool plan_skinny(int rows, const Geometry& g, int epi, bool gemv, SkinnyPlan& p) {
+    const int forced = switch_value(SW_SKINNY);
+    if (forced == 0 || rows > SKINNY_MAX_ROWS || switch_value(SW_GEMM_VARIANT) >= 0 || switch_value(SW_SPLITS) > 0)
+        return false;
+    const int cus = device_cus();
+    p.row_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : 8;
+    const int groups = (rows + 16 * p.row_tiles - 1) / (16 * p.row_tiles);
+    p.col_tiles = epi != EPI_PLAIN || g.N_pad / 16 * groups > cus ? 2 : 1;
+    p.blocks_n = g.N_pad / (16 * p.col_tiles);
+    if (forced > 0) return true;
+    if (gemv && (rows <= 2 || (rows <= 4 && g.bits == 8))) return false;
+    if (rows <= 64) return true;
+    const size_t per_cu = ((size_t)p.blocks_n * groups + cus - 1) / cus;
+    return per_cu * 16 * p.row_tiles * g.K_pad <= skinny_code_bytes;
+}
+
 // --- workspaces -------------------------------------------------------------
 
 struct WsLayout {
@@ -462,7 +501,10 @@ static WsLayout ws_layout(const Geometry& g, int M) {
     L.codes = (size_t)(g.K_pad / 16) * M_alloc * 16;
     L.rows = round_up_z((size_t)M_alloc * 4, 256);
     L.c = round_up_z((size_t)M * g.N * 4, 256);
-    L.part = round_up_z((size_t)8 * (g.N_pad / 8) * 4, 256);
+    // one GEMV row maximum per 8 columns (up to 8 rows), or skinny_kernel's per
+    // pair of 16-column tiles
+    const size_t skinny_rows = g.half ? std::min(M, SKINNY_MAX_ROWS) : 0;
+    L.part = round_up_z(std::max((size_t)g.N_pad, skinny_rows * (g.N_pad / 32)) * 4, 256);
     L.split_part_ints = split_need(g, M);
     L.split_part = round_up_z(L.split_part_ints * 4, 256);
     L.kacc = round_up_z(((size_t)g.N_pad + 8) * 8, 256);
@@ -646,7 +688,9 @@ int enqueue_linear(Workspace* ws, const Weights* w, const void* x, int x_type, l
     const Geometry& g = w->g;
     if (comb && comb->combined) *comb->combined = false;
     const Plan pv = plan_linear(rows, g);
-    if (pv.kind == 0) {
+    SkinnyPlan sk;
+    const bool skinny = plan_skinny(rows, g, epi, pv.kind == 0, sk);
+    if (pv.kind == 0 && !skinny) {
         GemvParams V{};
         V.x = x;
         V.lda = lda;
@@ -746,7 +790,8 @@ int enqueue_linear(Workspace* ws, const Weights* w, const void* x, int x_type, l
         prof_end(slot, s);
         if (out_max) *out_max = RowMax{ws->partmax, grid};
     } else {
-        int rc = enqueue_quant(ws, x, x_type, lda, rows, rule, in_max, epi != EPI_PLAIN ? ws->rowmax : nullptr, s);
+        int rc = enqueue_quant(ws, x, x_type, lda, rows, rule, in_max,
+                               epi != EPI_PLAIN && !skinny ? ws->rowmax : nullptr, s);
         if (rc != RK_NPU_OK) return rc;
         const size_t c_esz = c_type == DT_F32 ? 4 : 2;
         const bool staged = (reinterpret_cast<uintptr_t>(c) & 15) == 0 && ((size_t)ldc * c_esz) % 16 == 0;
@@ -780,6 +825,15 @@ int enqueue_linear(Workspace* ws, const Weights* w, const void* x, int x_type, l
         G.splits = p.ksplit;
         G.split_part = ws->split_part;
         char name[64];
+        if (skinny) {
+            std::snprintf(name, sizeof(name), "skinny<%dx%d,w%d,epi=%d>", 16 * sk.row_tiles, 16 * sk.col_tiles, g.bits,
+                          epi);
+            const int slot = prof_begin(s, 1, g.bits, epi, rows, g.K, g.N, name);
+            launch_skinny(g.bits, epi, sk, staged, G, out_max ? ws->partmax : nullptr, s);
+            prof_end(slot, s);
+            if (out_max) *out_max = RowMax{ws->partmax, sk.blocks_n};
+            return hipGetLastError() == hipSuccess ? RK_NPU_OK : RK_NPU_ERR_DEVICE;
+        }
         std::snprintf(name, sizeof(name), "gemm<%dx%d,w%d,epi=%d,k/%d>", p.bm, p.bn, g.bits, epi, p.ksplit);
         const int slot = prof_begin(s, 1, g.bits, epi, rows, g.K, g.N, name);
         launch_gemm_any(g.bits, epi, p.variant, staged, G, p.tiles, s);

@@ -24,6 +24,17 @@ enum GemmVariant { V256x256 = 0, V256x128 = 1, V128x128 = 2, V64x128 = 3, V32x12
 void launch_gemm_w8(int epi, int v, bool staged, const GemmParams& G, int tiles, hipStream_t s);
 void launch_gemm_w4(int epi, int v, bool staged, const GemmParams& G, int tiles, hipStream_t s);
 
+// skinny_kernel over blocks of 16 * row_tiles rows and col_tiles 16-column
+// tiles (SwiGLU: a gate and an up tile). part: the SwiGLU row maxima
+// [row][blocks_n], or nullptr.
+struct SkinnyPlan {
+    int row_tiles;  // 1, 2, 4 or 8
+    int col_tiles;  // 1 or 2
+    int blocks_n;   // blocks along the columns
+};
+void launch_skinny(int bits, int epi, const SkinnyPlan& p, bool staged, const GemmParams& G, float* part,
+                   hipStream_t s);
+
 // GEMV of `mr` rows (1, 2, 4, 8), rows quantized beforehand (preq), by a
 // quantization wave (qwn = 1) or by the block; split-K pieces; the one-row
 // plain GEMV with the MoE combine (f32 activations only).

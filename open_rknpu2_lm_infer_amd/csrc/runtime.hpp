@@ -103,7 +103,7 @@ struct Workspace {
     int* rowsum;      // [M_alloc]
     unsigned* rowmax; // [M_alloc]  max|middle| of a fused SwiGLU output
     float* c_f32;     // [M][N]   output staging / fused middle
-    float* partmax;   // [8][N_pad/8] per-block max|middle| of a GEMV SwiGLU
+    float* partmax;   // per-block max|middle| of a GEMV's ([8][N_pad/8]) or skinny_kernel's SwiGLU
     int* split_part;        // split-K int32 partials [pieces][tiles][tile ints]
     size_t split_part_ints; // partial ints available
     unsigned long long* kacc;  // split-K GEMV column slots [N_pad] + row code-sum slot, kept zero between calls

@@ -1,0 +1,115 @@
+"""The streaming kernel for few rows (skinny_kernel): equal to the oracle at
+the edges of its tiles, and to the path it takes calls from in every form the
+device entries accept (types, unaligned buffers, ragged sizes, the fused FFN,
+the allocation-free entry). Bit for bit: the sums are exact integers and the
+dequantization is the same sequence of single-rounding operations."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle
+from open_rknpu2_lm_infer_amd import _ffi as F
+from open_rknpu2_lm_infer_amd import device as D
+from open_rknpu2_lm_infer_amd import npu
+from tests import refdata as R
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return D.DeviceContext(8)
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# K: one unit; an odd count of W4 planes (640 + 64, 100 -> 128, 12000 -> 12032);
+# the narrow window's last unit and the wide one's first; more units than the
+# wide window holds (reloaded). N: one tile, ragged and padded columns, two
+# column tiles per block (more than 4096 columns).
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("k,n", [(64, 16), (100, 100), (704, 768), (2560, 320), (2624, 1003), (12000, 64), (192, 4352)])
+def test_skinny_matches_oracle(ctx, bits, k, n):
+    codes, scales = R.weights(21, f"sk{bits}-{k}-{n}", bits, k, n)
+    w = ctx.weights(bits, dev(codes), dev(scales))
+    for rows in (2, 5, 8, 16, 17, 32, 33, 64, 65, 128, 129, 256):
+        x = R.activations(21, f"sk-x{rows}-{k}", rows, k)
+        for swiglu in (False, True)[:2 if n % 64 == 0 else 1]:
+            want = oracle.linear_swiglu(codes, scales, x) if swiglu else oracle.linear(codes, scales, x)
+            print(f"W{bits} K={k} N={n} rows={rows} swiglu={swiglu}", flush=True)
+            y = torch.full(want.shape, float("nan"), device="cuda")
+            with D.plan_switch("HM_SKINNY", 1):
+                D.linear(ctx, w, dev(x), y, rows, swiglu=swiglu)
+            torch.cuda.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [3, 8, 20, 70])
+def test_skinny_equals_the_other_path_in_every_form(ctx, bits, rows):
+    """Input and output types, bases off 16-byte alignment, K and N off every
+    multiple: HM_SKINNY 1 against 0."""
+    for k, n in ((512, 320), (333, 321)):
+        codes, scales = R.weights(22, f"skf{bits}-{k}-{n}", bits, k, n)
+        w = ctx.weights(bits, dev(codes), dev(scales))
+        x = R.activations(22, f"skf-x{rows}-{k}", rows, k)
+        for swiglu in (False, True)[:2 if n % 64 == 0 else 1]:
+            width = n // 2 if swiglu else n
+            for x_type in (torch.float16, torch.float32):
+                for y_type in (torch.float16, torch.float32):
+                    for off in (0, 1):
+                        xb = torch.zeros(rows * k + off, dtype=x_type, device="cuda")
+                        xin = xb[off:].view(rows, k)
+                        xin.copy_(dev(x))
+                        got = []
+                        for skinny in (1, 0):
+                            buf = torch.zeros(rows * width + off, dtype=y_type, device="cuda")
+                            with D.plan_switch("HM_SKINNY", skinny):
+                                D.linear(ctx, w, xin, buf[off:].view(rows, width), rows, swiglu=swiglu)
+                            torch.cuda.synchronize()
+                            got.append(buf.cpu())
+                        assert torch.equal(got[0], got[1]), (k, n, swiglu, x_type, y_type, off)
+
+
+@pytest.mark.parametrize("rows", [4, 8, 16, 40, 64, 130, 256])
+@pytest.mark.parametrize("gu_bits,dn_bits", [(4, 4), (4, 8), (8, 8)])
+def test_skinny_ffn_row_maxima(ctx, rows, gu_bits, dn_bits):
+    """The middle's row maxima pass from the gate_up launch to the
+    requantization as one partial per block (f = 2080: 130 blocks), whichever
+    of the two launches runs on which kernel; three calls in a row."""
+    h, f = 384, 2080
+    gc, gs = R.weights(23, f"skg{gu_bits}", gu_bits, h, 2 * f)
+    dc, ds = R.weights(23, f"skd{dn_bits}", dn_bits, f, h)
+    gu, dn = ctx.weights(gu_bits, dev(gc), dev(gs)), ctx.weights(dn_bits, dev(dc), dev(ds))
+    for rep, skinny in enumerate((1, -1, 0)):
+        x = R.activations(23, f"skffn-x{rows}-{rep}", rows, h)
+        y = torch.empty(rows, h, dtype=torch.float32, device="cuda")
+        with D.plan_switch("HM_SKINNY", skinny):
+            D.ffn(ctx, gu, dn, dev(x), y, rows)
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), oracle.ffn(gc, gs, dc, ds, x)), skinny
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [8, 16, 100, 256])
+def test_skinny_static_entry(ctx, bits, rows):
+    """rk_npu_hip_linear_run_static (no workspace): the same result, plain
+    and SwiGLU (which wants no row maxima there)."""
+    k, n = 640, 512
+    codes, scales = R.weights(24, f"sks{bits}", bits, k, n)
+    w = ctx.weights(bits, dev(codes), dev(scales))
+    x = R.activations(24, f"sks-x{rows}", rows, k)
+    xd = dev(x)
+    for epi, width, want in ((F.RK_NPU_HIP_PLAIN, n, oracle.linear(codes, scales, x)),
+                             (F.RK_NPU_HIP_SWIGLU, n // 2, oracle.linear_swiglu(codes, scales, x))):
+        y = torch.empty(rows, width, device="cuda")
+        npu.check(F.lib().rk_npu_hip_linear_run_static(w.handle.raw, bits, ctypes.c_void_p(xd.data_ptr()),
+                                                       F.RK_NPU_HIP_F32, ctypes.c_void_p(y.data_ptr()),
+                                                       F.RK_NPU_HIP_F32, rows, epi, D.current_stream()), "static")
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy(), want)
