@@ -941,20 +941,26 @@ static int cache_put(AttnCache* c, const void* k, const void* v, int rows, hipMe
     return RK_NPU_OK;
 }
 
-// Host-buffer append: rows of K and V ([kv_heads][rows][D] each, V at
-// byte offset voff of the stage) copied into the cache rows [length, length +
-// rows) of every head, 16 bytes per thread and step.
-__global__ __launch_bounds__(256) void attn_append_kernel(const v4u* __restrict__ src, size_t voff_pieces,
-                                                          v4u* __restrict__ k, v4u* __restrict__ v, int rows,
-                                                          int row_pieces, size_t head_pieces, int length,
-                                                          size_t total) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-        const size_t per_head = (size_t)rows * row_pieces;
-        const size_t h = i / per_head, r = i % per_head;
-        const size_t at = h * head_pieces + (size_t)length * row_pieces + r;
-        k[at] = src[i];
-        v[at] = src[voff_pieces + i];
-    }
+// Append: rows of K (blockIdx.z 0) and V (1), [kv_heads][rows][D] each, into
+// the rows [length, length + rows) of every head (blockIdx.y), 16 bytes per
+// thread and step. One launch where two 2-D copies took one each (a decode
+// step's two copies 4.5 us apiece on the stream).
+__global__ __launch_bounds__(256) void attn_append_kernel(const v4u* __restrict__ ksrc, const v4u* __restrict__ vsrc,
+                                                          v4u* __restrict__ k, v4u* __restrict__ v, int pieces,
+                                                          size_t head_pieces, size_t first) {
+    const v4u* src = (blockIdx.z ? vsrc : ksrc) + (size_t)blockIdx.y * pieces;
+    v4u* dst = (blockIdx.z ? v : k) + (size_t)blockIdx.y * head_pieces + first;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < pieces; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+// Launches it for `rows` rows whose K and V lie at 16-byte aligned device (or
+// mapped host) addresses; the caller advances the length.
+static void enqueue_append(AttnCache* c, const void* k, const void* v, int rows, hipStream_t s) {
+    const int row_pieces = c->cfg.head_dim / 8, pieces = rows * row_pieces;
+    hipLaunchKernelGGL(attn_append_kernel, dim3(std::min(1024, (pieces + 255) / 256), c->cfg.kv_heads, 2), dim3(256), 0,
+                       s, static_cast<const v4u*>(k), static_cast<const v4u*>(v), reinterpret_cast<v4u*>(c->k),
+                       reinterpret_cast<v4u*>(c->v), pieces, (size_t)c->capacity * row_pieces,
+                       (size_t)c->length * row_pieces);
 }
 
 // Appends host rows through the cache's pinned stage and stream, returning
@@ -973,12 +979,7 @@ static bool cache_put_staged(AttnCache* c, const void* k, const void* v, int row
     if (!st) return false;
     std::memcpy(st, k, each);
     std::memcpy(static_cast<uint8_t*>(st) + voff, v, each);
-    const int row_pieces = D / 8;
-    const size_t total = (size_t)kh * rows * row_pieces;
-    const int blocks = (int)std::min<size_t>(1024, (total + 255) / 256);
-    hipLaunchKernelGGL(attn_append_kernel, dim3(blocks), dim3(256), 0, c->stream, static_cast<const v4u*>(c->hs.dev),
-                       voff / 16, reinterpret_cast<v4u*>(c->k), reinterpret_cast<v4u*>(c->v), rows, row_pieces,
-                       (size_t)c->capacity * row_pieces, c->length, total);
+    enqueue_append(c, c->hs.dev, static_cast<const uint8_t*>(c->hs.dev) + voff, rows, c->stream);
     if (hipGetLastError() != hipSuccess || !stage_download(c->hs, true, st, nullptr, nullptr, 0, c->stream)) {
         (void)hipStreamSynchronize(c->stream);
         rc = RK_NPU_ERR_DEVICE;
@@ -1381,7 +1382,14 @@ int rk_npu_hip_attention_cache_append(rk_npu_attention_f16_cache* cache, const v
     if (!c || rows < 1 || !k_dev || !v_dev) return RK_NPU_ERR_PARAM;
     if ((long)c->length + rows > c->capacity) return RK_NPU_ERR_PARAM;  // (reserve first: no allocation here)
     if (hipSetDevice(device_of(c->domain)) != hipSuccess) return RK_NPU_ERR_DEVICE;
-    const int rc = cache_put(c, k_dev, v_dev, rows, hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream), true);
+    int rc;
+    if (((reinterpret_cast<uintptr_t>(k_dev) | reinterpret_cast<uintptr_t>(v_dev)) & 15) == 0) {
+        enqueue_append(c, k_dev, v_dev, rows, static_cast<hipStream_t>(stream));
+        rc = hipGetLastError() == hipSuccess ? RK_NPU_OK : RK_NPU_ERR_DEVICE;
+        if (rc == RK_NPU_OK) c->length += rows;
+    } else {
+        rc = cache_put(c, k_dev, v_dev, rows, hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream), true);
+    }
     if (rc == RK_NPU_OK) c->fence.note(static_cast<hipStream_t>(stream));
     return rc;
 }

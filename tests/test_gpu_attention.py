@@ -333,3 +333,37 @@ def test_host_poll_fallback_appends_and_runs():
     att = be.attention(qh, kh, d, scale)
     with D.plan_switch("HM_HOST_POLL", 0):
         run_sequence(att, qh, kh, d, (100, 1, 1, 2), np.random.default_rng(12), scale)
+
+
+def test_device_append_unaligned_source():
+    """Source rows off 16-byte alignment are copied like aligned ones."""
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=64))
+    qh, kh, d, rows = 4, 2, 64, 9
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = qh, kh, d, d ** -0.5
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, 64, 64
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    try:
+        g = torch.Generator(device="cuda").manual_seed(3)
+        buf = torch.randn(2 * kh * rows * d + 1, generator=g, device="cuda").half()
+        q = torch.randn(qh, rows, d, generator=g, device="cuda").half()
+        outs = []
+        for off in (0, 1):
+            src = torch.empty(buf.numel() + 8, dtype=torch.float16, device="cuda")
+            src[off:off + buf.numel()] = buf
+            out = torch.empty(qh, rows, d, device="cuda")
+            stream = torch.cuda.current_stream().cuda_stream
+            npu.check(L.rk_npu_attention_f16_cache_truncate(cache, 0), "truncate")
+            npu.check(L.rk_npu_hip_attention_cache_append(cache, src[off:].data_ptr(),
+                                                          src[off + kh * rows * d:].data_ptr(), rows, stream), "append")
+            npu.check(L.rk_npu_hip_attention_run(ws, cache, q.data_ptr(), rows, 0, out.data_ptr(), 0, stream), "run")
+            torch.cuda.synchronize()
+            outs.append(out.cpu())
+        assert torch.equal(*outs)
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
