@@ -12,9 +12,11 @@
 // Work split: block = (key split, tile of RT query rows, KV head). The query
 // rows of one KV head are its (query head of the group, query row) pairs, so
 // the group's heads share every K/V tile read. A block streams 64-key tiles
-// of K then V through LDS; a decode-sized call (few rows) spreads the keys
-// over many splits whose partial (max, sum, accumulators) a second launch
-// combines.
+// of K and V through LDS; where the rows give fewer blocks than CUs, the keys
+// are spread over splits whose partial (max, sum, accumulators) a second
+// launch combines. Three kernels (plan_attention): attn_tile_kernel, the
+// general one; attn_wide_kernel, many rows over many keys; attn_split_kernel,
+// a row or four of head_dim 256 over few keys.
 
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
@@ -30,6 +32,7 @@
 #pragma clang diagnostic ignored "-Wunused-function"  // (the header's other kernels)
 #include "kernels.hpp"
 #pragma clang diagnostic pop
+#include "launch.hpp"
 #include "runtime.hpp"
 
 namespace hm {
@@ -38,9 +41,9 @@ constexpr uint32_t MAGIC_ATTN_CACHE = 0x43414841u;
 constexpr uint32_t MAGIC_ATTN_WORK = 0x57414841u;
 constexpr int ATTN_KT = 64;              // keys per tile
 constexpr int ATTN_MAX_SPLITS = 256;     // key splits per (KV head, row tile)
-// Partial rows a workspace holds: plan_attention launches at most 2048
-// blocks when it splits the keys, each with at most 128 query rows (head_dim
-// 64 and 128, MFMA tiles) or 16 (head_dim 256).
+// Partial rows a workspace holds: when it splits the keys, plan_attention
+// launches fewer than 512 blocks of 64 or 128 query rows, or 1024 of 32 or 4
+// (head_dim 256: 64 rows at most).
 static inline size_t attn_partial_rows(int head_dim) { return (size_t)2048 * (head_dim <= 128 ? 64 : 16); }
 
 struct AttnParams {
@@ -54,6 +57,7 @@ struct AttnParams {
     float scale;
     int splits, keys_per_split, row_tiles, key_end;
     int rows_pad;     // row_tiles * RT: partial rows per KV head
+    float max_unit;   // the partials' maxima in powers of 2: 1 (base 2) or log2(e) (natural)
 };
 
 // max / sum over the N consecutive lanes (N = 16 or 64) that share a query row
@@ -86,27 +90,29 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
-// Block: 256 threads; RT query rows (RT = 4: 64 threads per row, RT = 16: 16
-// threads per row). Thread (row, sub) scores keys sub + RPT*i of each tile
-// and owns output dims [sub*DPT, sub*DPT + DPT) of its row. K/V tiles (64
-// keys, 32 at head_dim 256) go through two LDS buffers; the next tile's loads
-// are in flight (registers) while the current tile is computed. Scores are
+// Block: 256 threads; RT query rows (4: 64 threads per row), head_dim 256.
+// Thread (row, sub) scores key sub of each tile and owns output dims
+// [sub*DPT, sub*DPT + DPT) of its row. K/V tiles of 32 keys go through LDS;
+// the next tile's loads are in flight (registers) while the current tile is
+// computed. Left for at most 4 rows over few keys, where it is launch and
+// latency: one row of 4-head groups over 1000 keys of 8 KV heads 8.7 us, on
+// attn_tile_kernel 9.2; over 300 7.2 and 8.3. Scores are
 // v_dot2_f32_f16 sums over the fp16 q and k pairs (exact products, f32
 // accumulation) times the scale; p * v folds the fp16 conversion into the
 // multiply-add.
 template <int D, int RT>
 __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    constexpr int KT = D == 256 ? 32 : ATTN_KT;      // keys per tile
+    constexpr int KT = 32;                           // keys per tile
     constexpr int RPT = 256 / RT;                    // threads per row
     constexpr int SPT = KT >= RPT ? KT / RPT : 1;    // scores per thread per tile
     constexpr int DPT = D / RPT;                     // output dims per thread
     constexpr int KP = D + 8;                        // LDS row pitch of a K/V tile (halves)
     constexpr int PER = (KT * (D / 8) + 255) / 256;  // 16-byte K (and V) pieces per thread per tile
     constexpr int QPT = RT * D / 256;                // q halves per thread (2..16)
-    static_assert(DPT >= 1 && D % RPT == 0 && D % 8 == 0 && (QPT == 1 || QPT % 2 == 0),
+    static_assert(DPT >= 1 && D % RPT == 0 && D % 8 == 0 && QPT % 2 == 0,
                   "head_dim must split over the threads");
-    constexpr int QW = QPT >= 2 ? QPT / 2 : 1;  // q words per thread (QPT = 1: one half)
+    constexpr int QW = QPT / 2;  // q words per thread
     __shared__ __attribute__((aligned(16))) __half qs[RT][D];
     __shared__ __attribute__((aligned(16))) __half ks[KT][KP];
     __shared__ __attribute__((aligned(16))) __half vs[KT][KP];
@@ -129,9 +135,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
     const __half* qsrc = P.q + ((size_t)(g * G + (q_ok ? qrr / P.m : 0)) * P.m + (q_ok ? qrr % P.m : 0)) * D + qcol;
     unsigned qv[QW];
 #pragma unroll
-    for (int i = 0; i < QW; ++i)
-        qv[i] = QPT == 1 ? (unsigned)reinterpret_cast<const unsigned short*>(qsrc)[0]
-                         : reinterpret_cast<const unsigned*>(qsrc)[i];
+    for (int i = 0; i < QW; ++i) qv[i] = reinterpret_cast<const unsigned*>(qsrc)[i];
     v4u kr[PER], vr[PER];
     auto issue = [&](int kb) {
 #pragma unroll
@@ -155,12 +159,8 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
         }
     };
     if (k0 < k1) issue(k0);
-    if constexpr (QPT == 1) {
-        reinterpret_cast<unsigned short*>(&qs[qrow][qcol])[0] = q_ok ? (unsigned short)qv[0] : (unsigned short)0;
-    } else {
 #pragma unroll
-        for (int i = 0; i < QW; ++i) reinterpret_cast<unsigned*>(&qs[qrow][qcol])[i] = q_ok ? qv[i] : 0u;
-    }
+    for (int i = 0; i < QW; ++i) reinterpret_cast<unsigned*>(&qs[qrow][qcol])[i] = q_ok ? qv[i] : 0u;
     float mrun = -INFINITY, lrun = 0.0f;
     float acc[DPT];
 #pragma unroll
@@ -240,10 +240,10 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
     for (int e = 0; e < DPT; ++e) part[2 + sub * DPT + e] = acc[e];
 }
 
-// Matrix-core variant for 16 or more query rows per KV head (head_dim 64 or
-// 128). Block = NW waves (4 or 8), each owning 16 query rows of one KV head, over
-// 64-key tiles of its key split; the K/V tile is shared by the block. Per
-// tile, with v_mfma_f32_16x16x32_f16 (fp16 operands, f32 accumulation):
+// Many rows over many keys (head_dim 64 or 128). Block = 8 waves, each owning
+// 16 query rows of one KV head, over 64-key tiles of its key split; the K/V
+// tile is shared by the block. Per tile, with v_mfma_f32_16x16x32_f16 (fp16
+// operands, f32 accumulation):
 //   S^T = K Q^T   A = K rows from LDS, B = Q fragments held in registers;
 //                 the accumulator gives lane l the raw scores of query row
 //                 l%16 for keys 4(l/16)..+3 of each 16-key block,
@@ -263,18 +263,16 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
 // (v_dot2 against ones: the fp16 weights summed exactly in f32), added over
 // the row's 4 lanes at the end. Masks (causal, keys past the split) apply
 // only on tiles that cross them.
-// Tiles reach LDS in one of two ways:
-//   8 waves (one block per CU): direct global->LDS loads into three tile
-//     buffers, K and V row-major (key, dim) in 16-byte slots permuted within
-//     each row against bank conflicts; tile t + 2 is requested after tile t's
-//     last LDS reads, into the buffer of tile t - 1 (every wave has passed
-//     tile t's barrier, so it is free), one barrier per tile; V^T fragments
-//     come from transposing LDS reads (ds_read_b64_tr_b16);
-//   4 waves (several blocks per CU, where 96 KB of tile buffers would leave
-//     one): the next tile's K/V in registers while this one is used, stored
-//     between two barriers, V transposed on the way in (each 32-key chunk's
-//     4-key groups in the order 0 4 1 5 2 6 3 7, so a lane's 8 k-slots are
-//     one 16-byte read).
+// Tiles reach LDS by direct global->LDS loads into three buffers, K and V
+// row-major (key, dim) in 16-byte slots permuted within each row against bank
+// conflicts; tile t + 2 is requested after tile t's last LDS reads, into the
+// buffer of tile t - 1 (every wave has passed tile t's barrier, so it is
+// free), one barrier per tile; V^T fragments come from transposing LDS reads
+// (ds_read_b64_tr_b16).
+// Against attn_tile_kernel, whose waves share a row group's keys: half the LDS
+// writes and barriers per row and key, but 128 rows per block and twice the
+// partial rows. 512 rows per KV head (8 heads of 128) over 4096 keys 25.0 us
+// here, 26.9 there; 1024 over 16128 94 and 128; 512 over 2028 20.6 and 19.0.
 // Operand layouts (16x16x32, wave64): A lane l = row l%16, k-slots
 // 8(l/16)..+7; B lane l = column l%16, same k-slots; C lane l = rows
 // 4(l/16)..+3 of column l%16.
@@ -298,8 +296,9 @@ __device__ __forceinline__ float sum_rows4(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int D, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
+constexpr int ATTN_WIDE_WAVES = 8;
+template <int D>
+__global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnParams P) {
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     typedef _Float16 hh2 __attribute__((ext_vector_type(2)));
     typedef float f4 __attribute__((ext_vector_type(4)));
@@ -307,24 +306,13 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
     typedef short s4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) s4 lds_s4;
     constexpr int KT = ATTN_KT, KS = D / 32, NB = D / 16;
-    constexpr int NT = 64 * NW;
-    constexpr bool DMA = NW == 8;
-    static_assert(D == 64 || D == 128, "MFMA attention: head_dim 64 or 128");
-    static_assert(KT == 64, "tile shape");
-    // direct loads: 16-byte slots per row, bytes of one matrix of a tile,
-    // slots per thread per matrix, tile buffers
+    constexpr int NW = ATTN_WIDE_WAVES, NT = 64 * NW;
+    // 16-byte slots per row, bytes of one matrix of a tile, slots per thread
+    // per matrix, tile buffers
     constexpr int SPR = D / 8, MAT = KT * D * 2, DPT = KT * SPR / NT, NBUF = 3;
-    static_assert(!DMA || KT * SPR % NT == 0, "tile shape");
-    // register path: row pads against LDS bank conflicts in the fragment
-    // reads (pads of 16 halves measured fastest), 16-byte K pieces per tile,
-    // V pieces of 4 keys x 8 dims per tile
-    constexpr int KP = D + 16, VP = KT + 16;
-    constexpr int KPIECES = KT * (D / 8), VPIECES = (KT / 4) * (D / 8), KPT = KPIECES / NT;
-    static_assert(DMA || (KPIECES % NT == 0 && VPIECES <= NT), "tile shape");
-    constexpr int SMEM = DMA ? NBUF * 2 * MAT : (KT * KP + D * VP) * 2;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM];
-    auto ks = reinterpret_cast<__half (*)[KP]>(smem);
-    auto vt = reinterpret_cast<__half (*)[VP]>(smem + KT * KP * 2);
+    static_assert(D == 64 || D == 128, "head_dim 64 or 128");
+    static_assert(KT == 64 && KT * SPR % NT == 0, "tile shape");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NBUF * 2 * MAT];
 
     const int split = blockIdx.x, rt = blockIdx.y, g = blockIdx.z;
     const int G = P.qh / P.kh, R = G * P.m;
@@ -361,7 +349,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
         }
     }
 
-    // --- direct loads. Slot c of row r lies at c ^ swk(r) (K: 16 consecutive
+    // Direct loads: slot c of row r lies at c ^ swk(r) (K: 16 consecutive
     // rows take 16 distinct slots of one logical column, which the score
     // fragments read per 16 lanes) or c ^ swv(r) (V: 8 consecutive rows take
     // distinct slot pairs 2c, 2c + 1, the 32 bytes of each of 8 rows a half
@@ -370,15 +358,13 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
     auto swv = [](int r) { return D == 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); };
     // this thread's slots: physical slot t * NT + tid of each matrix -> row,
     // and the logical slot (16-byte column) it holds
-    int drow[DMA ? DPT : 1], dkc[DMA ? DPT : 1], dvc[DMA ? DPT : 1];
-    if constexpr (DMA) {
+    int drow[DPT], dkc[DPT], dvc[DPT];
 #pragma unroll
-        for (int t = 0; t < DPT; ++t) {
-            const int pslot = t * NT + tid, r = pslot / SPR, ps = pslot % SPR;
-            drow[t] = r;
-            dkc[t] = ps ^ swk(r);
-            dvc[t] = ps ^ swv(r);
-        }
+    for (int t = 0; t < DPT; ++t) {
+        const int pslot = t * NT + tid, r = pslot / SPR, ps = pslot % SPR;
+        drow[t] = r;
+        dkc[t] = ps ^ swk(r);
+        dvc[t] = ps ^ swv(r);
     }
     // keys past the split read the split's last key (finite data; masked)
     auto issue_dma = [&](int kb, int buf) {
@@ -394,106 +380,22 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
         }
     };
 
-    // --- register path. K piece i: key i / (D/8), dims 8 (i % (D/8)); V
-    // piece (tid): keys 4 (tid % 16)..+3, dims 8 (tid / 16)..+7
-    const bool vthread = tid < VPIECES;
-    const int vj = tid & 15, vc = tid >> 4;
-    // byte offsets within a tile (the tile base is uniform): K piece t, V row t
-    unsigned koff[DMA ? 1 : KPT], voff[4];
-    v4u kr[DMA ? 1 : KPT], vr[4];
-    if constexpr (!DMA) {
-#pragma unroll
-        for (int t = 0; t < KPT; ++t) {
-            const int i = tid + NT * t;
-            koff[t] = (unsigned)((i / (D / 8)) * D + (i % (D / 8)) * 8) * 2u;
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) voff[t] = (unsigned)((4 * vj + t) * D + vc * 8) * 2u;
-    }
-    auto issue_regs = [&](int kb) {
-        const char* kt = reinterpret_cast<const char*>(kbase + (size_t)kb * D);
-        const char* vtp = reinterpret_cast<const char*>(vbase + (size_t)kb * D);
-        if (kb + KT <= k1) {  // (uniform) whole tile inside the split
-#pragma unroll
-            for (int t = 0; t < KPT; ++t) kr[t] = *reinterpret_cast<const v4u*>(kt + koff[t]);
-            if (vthread) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) vr[t] = *reinterpret_cast<const v4u*>(vtp + voff[t]);
-            }
-        } else {  // keys past the split read the tile's first row (zeroed in store)
-#pragma unroll
-            for (int t = 0; t < KPT; ++t) {
-                const int key = kb + (tid + NT * t) / (D / 8);
-                kr[t] = *reinterpret_cast<const v4u*>(kt + (key < k1 ? koff[t] : 0u));
-            }
-            if (vthread) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int key = kb + 4 * vj + t;
-                    vr[t] = *reinterpret_cast<const v4u*>(vtp + (key < k1 ? voff[t] : 0u));
-                }
-            }
-        }
-    };
-    auto store_regs = [&](int kb) {
-        if (kb + KT > k1) {  // (block-uniform) zero the keys past the split
-#pragma unroll
-            for (int t = 0; t < KPT; ++t)
-                if (kb + (tid + NT * t) / (D / 8) >= k1) kr[t] = v4u{0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                if (kb + 4 * vj + t >= k1) vr[t] = v4u{0u, 0u, 0u, 0u};
-        }
-#pragma unroll
-        for (int t = 0; t < KPT; ++t) {
-            const int i = tid + NT * t;
-            *reinterpret_cast<v4u*>(&ks[i / (D / 8)][(i % (D / 8)) * 8]) = kr[t];
-        }
-        if (vthread) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int cw = e >> 1;
-                u2 x;
-                if (e & 1) {
-                    x[0] = (vr[0][cw] >> 16) | (vr[1][cw] & 0xffff0000u);
-                    x[1] = (vr[2][cw] >> 16) | (vr[3][cw] & 0xffff0000u);
-                } else {
-                    x[0] = (vr[0][cw] & 0xffffu) | (vr[1][cw] << 16);
-                    x[1] = (vr[2][cw] & 0xffffu) | (vr[3][cw] << 16);
-                }
-                const int lg = vj & 7, pos = lg < 4 ? 2 * lg : 2 * lg - 7;
-                *reinterpret_cast<u2*>(&vt[vc * 8 + e][32 * (vj >> 3) + 4 * pos]) = x;
-            }
-        }
-    };
-
     f4 o[NB];
 #pragma unroll
     for (int n = 0; n < NB; ++n) o[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float mrun = -INFINITY, lpart = 0.0f;
     const hh2 ones = {(_Float16)1.0f, (_Float16)1.0f};
-    if constexpr (DMA) {
-        if (k0 < k1) issue_dma(k0, 0);
-        if (k0 + KT < k1) issue_dma(k0 + KT, 1);
-    } else {
-        if (k0 < k1) issue_regs(k0);
-    }
+    if (k0 < k1) issue_dma(k0, 0);
+    if (k0 + KT < k1) issue_dma(k0 + KT, 1);
     int buf = 0;
     for (int kb = k0; kb < k1; kb += KT) {
         const uint8_t* kst = smem + buf * 2 * MAT;
         const uint8_t* vst = kst + MAT;
-        if constexpr (DMA) {
-            if (kb + KT < k1)
-                wait_vmcnt<2 * DPT>();  // (this thread's loads of the tile have landed; the next tile's may not)
-            else
-                wait_vmcnt<0>();
-            __syncthreads();  // (every thread's have)
-        } else {
-            __syncthreads();  // (the previous tile's LDS reads are done)
-            store_regs(kb);
-            __syncthreads();
-            if (kb + KT < k1) issue_regs(kb + KT);
-        }
+        if (kb + KT < k1)
+            wait_vmcnt<2 * DPT>();  // (this thread's loads of the tile have landed; the next tile's may not)
+        else
+            wait_vmcnt<0>();
+        __syncthreads();  // (every thread's have)
         // (k outermost: the 4 key blocks' products are independent, so they
         // issue back to back instead of waiting on each other)
         f4 sacc[4];
@@ -502,9 +404,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
         for (int k = 0; k < KS; ++k)
 #pragma unroll
             for (int cb = 0; cb < 4; ++cb) {
-                const void* src = DMA ? static_cast<const void*>(kst + (cb * 16 + lo) * (D * 2) +
-                                                                ((4 * k + hi) ^ swk(lo)) * 16)
-                                      : static_cast<const void*>(&ks[cb * 16 + lo][32 * k + 8 * hi]);
+                const void* src = kst + (cb * 16 + lo) * (D * 2) + ((4 * k + hi) ^ swk(lo)) * 16;
                 ka[cb][k] = __builtin_bit_cast(h8, *reinterpret_cast<const v4u*>(src));
             }
 #pragma unroll
@@ -561,32 +461,26 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
             h8 va[NB];
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
-                if constexpr (DMA) {
-                    // transposing reads: lane j of a 16-lane group names dims
-                    // 4 (j % 4)..+3 of key row 4 (j / 4) of the group's 16
-                    // keys; lane i receives dim i of the rows named by lanes
-                    // i / 4, 4 + i / 4, 8 + i / 4, 12 + i / 4: its dim of keys
-                    // 4 hi..+3 (then of keys 16 + 4 hi..+3) of the step
-                    const int vr0 = 32 * k + 4 * hi + (lo >> 2);
-                    const uint8_t* p =
-                        vst + vr0 * (D * 2) + (((2 * n + ((lo & 3) >> 1)) ^ swv(vr0)) * 16) + (lo & 1) * 8;
-                    const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
-                    const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 16 * (D * 2)));
-                    const u2 ua = __builtin_bit_cast(u2, a), ub = __builtin_bit_cast(u2, b);
-                    va[n] = __builtin_bit_cast(h8, v4u{ua[0], ua[1], ub[0], ub[1]});
-                } else {
-                    va[n] = __builtin_bit_cast(h8, *reinterpret_cast<const v4u*>(&vt[16 * n + lo][32 * k + 8 * hi]));
-                }
+                // transposing reads: lane j of a 16-lane group names dims
+                // 4 (j % 4)..+3 of key row 4 (j / 4) of the group's 16
+                // keys; lane i receives dim i of the rows named by lanes
+                // i / 4, 4 + i / 4, 8 + i / 4, 12 + i / 4: its dim of keys
+                // 4 hi..+3 (then of keys 16 + 4 hi..+3) of the step
+                const int vr0 = 32 * k + 4 * hi + (lo >> 2);
+                const uint8_t* p =
+                    vst + vr0 * (D * 2) + (((2 * n + ((lo & 3) >> 1)) ^ swv(vr0)) * 16) + (lo & 1) * 8;
+                const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
+                const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 16 * (D * 2)));
+                const u2 ua = __builtin_bit_cast(u2, a), ub = __builtin_bit_cast(u2, b);
+                va[n] = __builtin_bit_cast(h8, v4u{ua[0], ua[1], ub[0], ub[1]});
             }
 #pragma unroll
             for (int n = 0; n < NB; ++n) o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[n], pb[k], o[n], 0, 0, 0);
         }
-        if constexpr (DMA) {
-            // (the compiler waits for every direct load in flight before a
-            // transposing read, so the request comes after this tile's)
-            if (kb + 2 * KT < k1) issue_dma(kb + 2 * KT, buf == 0 ? NBUF - 1 : buf - 1);
-            buf = buf == NBUF - 1 ? 0 : buf + 1;
-        }
+        // (the compiler waits for every direct load in flight before a
+        // transposing read, so the request comes after this tile's)
+        if (kb + 2 * KT < k1) issue_dma(kb + 2 * KT, buf == 0 ? NBUF - 1 : buf - 1);
+        buf = buf == NBUF - 1 ? 0 : buf + 1;
     }
     float l = lpart;
     l = sum_rows4(l);
@@ -610,10 +504,277 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
             }
         }
     } else {
-        // partial: running max in natural-log units as the combine expects
         float* part = P.part + (((size_t)g * P.rows_pad + rr) * P.splits + split) * (D + 2);
         if (hi == 0) {
-            part[0] = (mrun == -INFINITY) ? -INFINITY : mrun * 0.6931471805599453f;
+            part[0] = mrun;
+            part[1] = l;
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[2 + 16 * n + 4 * hi + r] = o[n][r];
+    }
+}
+
+// The general kernel: block = WR x WK waves; wave (wr, wk) owns 16 query rows
+// of one KV head and, of every stage of 32 WK keys, the 32 keys 32 wk..+31, so
+// WK waves share a row group's keys and their partial (max, sum, accumulators)
+// meet in LDS at the end; waves whose rows or keys are all masked skip their
+// products. Operands and lane layouts are attn_wide_kernel's: S^T = K Q^T,
+// softmax in place, O^T += V^T P^T with transposing V reads. Stages go global -> registers -> one of two LDS buffers: stage
+// t + 1 is in registers while stage t is computed, then stored to the buffer
+// stage t - 1 left (every wave passed the barrier after it), one barrier per
+// stage.
+//
+// SPLIT: the softmax weights keep f32's precision on the fp16 matrix cores as
+// a sum of two fp16 (p = ph + pl, pl = the rounded remainder: 22 bits of p),
+// two products per V fragment into the same accumulator, and the weights' sum
+// is taken in f32 before the split. They are scaled by 2^ATTN_SHIFT (which
+// leaves in the division), so that with the lazy maximum p stays below 2^15
+// and what the remainder loses below fp16's smallest value is 2^-32 of the
+// row's largest weight. Against 64 bits the outputs are nearer than the VALU
+// kernels' whose place this took (f32 weights, v_dot2 scores): 128 rows of 8-head
+// groups of 256 over 2048 keys 3.0e-7 (5.8e-7), one row of 128 over 16000
+// 2.9e-7 (4.4e-7). Calls that had fp16 weights keep them (SPLIT = false).
+//
+// Measured per run with its combine, us, the kernels before -> this (one row =
+// one query row, so 4 or 8 rows per KV head):
+//   head_dim 256, 16 heads / 2 KV, 128 rows x 2048 keys       112.5 -> 25.7
+//                 64 / 8, 128 rows x 8128                      1633 -> 138
+//                 16 / 2, 1 row x 16000                        26.0 -> 14.8
+//   head_dim 128, 32 / 8, 1 row x 3968                          9.1 ->  8.4
+//                 16 / 8, 1 row x 16000                        20.6 -> 16.6
+//                 32 / 8, 3 rows x 3970                        14.1 ->  9.3
+//                 32 / 8, 16 rows x 4016                       17.6 -> 14.4
+//                 32 / 8, 32 rows x 2032                       17.9 -> 13.5
+//   head_dim 64,  16 / 8, 1 row x 16000                        14.4 ->  9.7
+// At few rows it is launches and one or two memory round trips; at many, the
+// LDS reads of a fragment per 16 rows, the exponentials and the products,
+// which the two waves of a SIMD overlap only in part (head_dim 256: 0.7 us per
+// 64 keys of a 64-row block). RW = 2 (a fragment read serves 32 rows) and
+// 4-wave blocks of 64 or 128 rows were slower at every size tried.
+constexpr float ATTN_SHIFT = 7.0f;
+
+template <int D, int WR, int WK, bool SPLIT>
+__global__ __launch_bounds__(64 * WR * WK) void attn_tile_kernel(AttnParams P) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    // (q and out of any element alignment)
+    typedef unsigned q16 __attribute__((ext_vector_type(4), aligned(2)));
+    typedef unsigned o8 __attribute__((ext_vector_type(2), aligned(2)));
+    typedef float o16 __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int KS = D / 32, NB = D / 16, NT = 64 * WR * WK, RT = 16 * WR;
+    constexpr int KT = 32 * WK;                     // keys per stage
+    constexpr int SPR = D / 8, MAT = KT * D * 2;    // 16-byte slots per row, bytes of K (V) per stage
+    constexpr int PT = KT * SPR / NT;               // slots per thread and matrix
+    // two stage buffers, and the merge's maxima and sums (its accumulators lie
+    // in the stage buffer that the last stage does not use)
+    constexpr int WAVES1 = (WK - 1) * WR, SMEM = 4 * MAT + WAVES1 * 512;
+    constexpr float SHIFT = SPLIT ? ATTN_SHIFT : 0.0f;
+    static_assert(KT * SPR % NT == 0 && SMEM <= 160 * 1024 && WAVES1 * NB * 1024 <= 2 * MAT, "stage shape");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[SMEM];
+
+    const int split = blockIdx.x, rt = blockIdx.y, g = blockIdx.z;
+    const int G = P.qh / P.kh, R = G * P.m;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave % WR, wk = wave / WR;
+    const int lo = lane & 15, hi = lane >> 4;
+    const int k0 = split * P.keys_per_split;
+    const int k1 = min(k0 + P.keys_per_split, P.key_end);
+    const float c = P.scale * 1.4426950408889634f;
+    const __half* kbase = P.k + (size_t)g * P.cap * D;
+    const __half* vbase = P.v + (size_t)g * P.cap * D;
+    // slot of (row, 16-byte column) in a K / V tile: permuted within the row
+    // as in attn_wide_kernel's tiles
+    auto swk = [](int r) { return D >= 128 ? (r & 15) : ((r >> 1) & 7); };
+    auto swv = [](int r) { return D >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); };
+
+    auto issue = [&](int kb, v4u (&kr)[PT], v4u (&vr)[PT]) {
+        const int last = k1 - 1 - kb;  // (keys past the split read its last key: finite data, masked)
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            const int i = t * NT + tid;
+            const size_t off = (size_t)(kb + min(i / SPR, last)) * D + (i % SPR) * 8;
+            kr[t] = *reinterpret_cast<const v4u*>(kbase + off);
+            vr[t] = *reinterpret_cast<const v4u*>(vbase + off);
+        }
+    };
+    auto store = [&](int buf, const v4u (&kr)[PT], const v4u (&vr)[PT]) {
+        uint8_t* dst = smem + buf * 2 * MAT;
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            const int i = t * NT + tid, r = i / SPR, col = i % SPR;
+            *reinterpret_cast<v4u*>(dst + r * (D * 2) + (col ^ swk(r)) * 16) = kr[t];
+            *reinterpret_cast<v4u*>(dst + MAT + r * (D * 2) + (col ^ swv(r)) * 16) = vr[t];
+        }
+    };
+
+    v4u kr[PT], vr[PT], k0r[PT], v0r[PT];
+    if (k0 < k1) issue(k0, k0r, v0r);
+    // this lane's query row, its key limit and Q fragments
+    const int rr = rt * RT + wr * 16 + lo;
+    const bool ok = rr < R;
+    int lim = 0;
+    if (ok) lim = P.causal ? min(P.len, P.pos + rr % P.m + 1) : P.len;
+    // keys below `open` are visible to every row of the wave (rows past R are
+    // discarded and do not count), keys from `seen` on to none. (causal: the
+    // rows' places in their heads run from `first` to `last`)
+    const int r0 = rt * RT + wr * 16, rows = min(16, R - r0);
+    int open = min(P.len, k1), seen = rows > 0 ? open : 0;
+    if (P.causal && rows > 0) {
+        const int at = r0 % P.m;
+        const bool one = at + rows <= P.m;  // (all of one head)
+        const int first = one ? at : 0, last = one ? at + rows - 1 : P.m - 1;
+        open = min(open, P.pos + first + 1);
+        seen = min(seen, P.pos + last + 1);
+    }
+    h8 qf[KS];
+    const __half* qp = P.q + ((size_t)(g * G + (ok ? rr / P.m : 0)) * P.m + (ok ? rr % P.m : 0)) * D;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const v4u x = ok ? v4u(*reinterpret_cast<const q16*>(qp + 32 * k + 8 * hi)) : v4u{0u, 0u, 0u, 0u};
+        qf[k] = __builtin_bit_cast(h8, x);
+    }
+    if (k0 + KT < k1) issue(k0 + KT, kr, vr);
+    if (k0 < k1) store(0, k0r, v0r);
+
+    f4 o[NB];
+    float mrun = -INFINITY, lpart = 0.0f;  // (mrun: the row's maximum less SHIFT)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) o[n] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    __syncthreads();
+    int buf = 0;
+    for (int kb = k0; kb < k1; kb += KT) {
+        const uint8_t* kst = smem + buf * 2 * MAT + wk * (32 * D * 2);
+        const uint8_t* vst = kst + MAT;
+        const int key0 = kb + 32 * wk;
+        if (key0 < seen) {  // (wave-uniform)
+            f4 sacc[2] = {f4{0.0f, 0.0f, 0.0f, 0.0f}, f4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb) {
+                    const h8 ka = __builtin_bit_cast(
+                        h8, *reinterpret_cast<const v4u*>(kst + (cb * 16 + lo) * (D * 2) + ((4 * k + hi) ^ swk(lo)) * 16));
+                    sacc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[k], sacc[cb], 0, 0, 0);
+                }
+            h8 ph, pl;
+            if (__builtin_expect(key0 + 32 > open, 0)) {  // (uniform) the tile crosses a mask
+#pragma unroll
+                for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = key0 + cb * 16 + 4 * hi + r;
+                        if (!(key < lim && key < k1)) sacc[cb][r] = -INFINITY;
+                    }
+            }
+            float lmax = -INFINITY;
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb)
+                lmax = __builtin_elementwise_maximum(
+                    __builtin_elementwise_maximum(lmax, __builtin_elementwise_maximum(sacc[cb][0], sacc[cb][1])),
+                    __builtin_elementwise_maximum(sacc[cb][2], sacc[cb][3]));
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(lmax * c > mrun + (ATTN_LAZY + SHIFT)) != 0, 0)) {
+                const float tm = max_rows4(lmax) * c - SHIFT;
+                float alpha = 1.0f;
+                if (tm > mrun + ATTN_LAZY) {
+                    alpha = __builtin_amdgcn_exp2f(mrun - tm);  // (0 from -inf)
+                    mrun = tm;
+                }
+                lpart *= alpha;
+#pragma unroll
+                for (int n = 0; n < NB; ++n) o[n] *= alpha;
+            }
+            const float msub = (mrun == -INFINITY) ? 0.0f : mrun;
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[cb][r], c, -msub));
+                    const _Float16 h = (_Float16)p;
+                    ph[cb * 4 + r] = h;
+                    if constexpr (SPLIT) {
+                        pl[cb * 4 + r] = (_Float16)(p - (float)h);
+                        lpart += p;
+                    } else {
+                        lpart += (float)h;
+                    }
+                }
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                // transposing reads (as attn_wide_kernel's)
+                const int r0 = 4 * hi + (lo >> 2);
+                const uint8_t* p = vst + r0 * (D * 2) + (((2 * n + ((lo & 3) >> 1)) ^ swv(r0)) * 16) + (lo & 1) * 8;
+                const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
+                const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(p + 16 * (D * 2)));
+                const u2 ua = __builtin_bit_cast(u2, a), ub = __builtin_bit_cast(u2, b);
+                const h8 va = __builtin_bit_cast(h8, v4u{ua[0], ua[1], ub[0], ub[1]});
+                o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o[n], 0, 0, 0);
+                if constexpr (SPLIT) o[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[n], 0, 0, 0);
+            }
+        }
+        if (kb + KT < k1) {
+            store(buf ^ 1, kr, vr);
+            if (kb + 2 * KT < k1) issue(kb + 2 * KT, kr, vr);
+            __syncthreads();
+        }
+        buf ^= 1;
+    }
+
+    if constexpr (WK > 1) {
+        // the key groups' partials: waves wk > 0 leave theirs in LDS, wave
+        // (wr, 0) adds them
+        // (the stage buffer `buf` is free: the last stage uses the other one)
+        uint8_t* acc1 = smem + buf * 2 * MAT;
+        float* ml1 = reinterpret_cast<float*>(smem + 4 * MAT) + lane;
+        if (wk > 0) {
+            const int w = (wk - 1) * WR + wr;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) *reinterpret_cast<f4*>(acc1 + ((w * NB + n) * 64 + lane) * 16) = o[n];
+            ml1[w * 128] = mrun;
+            ml1[w * 128 + 64] = lpart;
+        }
+        __syncthreads();
+        if (wk > 0) return;
+#pragma unroll
+        for (int g1 = 1; g1 < WK; ++g1) {
+            const int w = (g1 - 1) * WR + wr;
+            const float m1 = ml1[w * 128], l1 = ml1[w * 128 + 64], m = fmaxf(mrun, m1);
+            const float a0 = mrun == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mrun - m);
+            const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - m);
+            mrun = m;
+            lpart = lpart * a0 + l1 * a1;
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+                o[n] = o[n] * a0 + *reinterpret_cast<const f4*>(acc1 + ((w * NB + n) * 64 + lane) * 16) * a1;
+        }
+    }
+    const float l = sum_rows4(lpart);
+    if (rr >= R) return;
+    if (P.splits == 1) {
+        const float inv = 1.0f / l;
+        const size_t o0 = ((size_t)(g * G + rr / P.m) * P.m + rr % P.m) * D + 4 * hi;
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const f4 y = o[n] * inv;
+            if (P.out_f16) {
+                const unsigned short b0 = __half_as_ushort(__float2half_rn(y[0]));
+                const unsigned short b1 = __half_as_ushort(__float2half_rn(y[1]));
+                const unsigned short b2 = __half_as_ushort(__float2half_rn(y[2]));
+                const unsigned short b3 = __half_as_ushort(__float2half_rn(y[3]));
+                *reinterpret_cast<o8*>(static_cast<__half*>(P.out) + o0 + 16 * n) =
+                    o8{b0 | ((unsigned)b1 << 16), b2 | ((unsigned)b3 << 16)};
+            } else {
+                *reinterpret_cast<o16*>(static_cast<float*>(P.out) + o0 + 16 * n) = y;
+            }
+        }
+    } else {
+        float* part = P.part + (((size_t)g * P.rows_pad + rr) * P.splits + split) * (D + 2);
+        if (hi == 0) {
+            part[0] = mrun;
             part[1] = l;
         }
 #pragma unroll
@@ -624,8 +785,9 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_kernel(AttnParams P) {
 }
 
 // Combine the key splits of one (KV head, row): block = (row, KV head).
-// Thread t takes split t for the max M and the weight w_t = exp(m_t - M) (0
-// for a split that saw no key) and the denominator sum_t w_t l_t; then wave w
+// Thread t takes split t for the max M and the weight w_t = e^(m_t - M) (or
+// 2^, as the maxima are kept: max_unit; 0 for a split that saw no key) and the
+// denominator sum_t w_t l_t; then wave w
 // takes splits w, w + 4, ... for all head dims (lane + 64 j), loading up to 16
 // splits at once so their latencies overlap; the 4 waves' sums meet in LDS:
 // out = sum_s w_s acc_s / sum_s w_s l_s.
@@ -660,7 +822,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams P) {
     if (lane == 0) red[0][wave] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-    const float w = (m == -INFINITY) ? 0.0f : __expf(m - mx);
+    const float w = (m == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * P.max_unit);
     w_s[tid] = w;
     const float den = group_sum<64>(w * l);
     if (lane == 0) red[1][wave] = den;
@@ -730,7 +892,7 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(AttnParams P) {
     const float m = lane < S ? p0[lane * STRIDE] : -INFINITY;
     const float l = lane < S ? p0[lane * STRIDE + 1] : 0.0f;
     const float mx = group_max<64>(m);
-    const float w = (m == -INFINITY) ? 0.0f : __expf(m - mx);
+    const float w = (m == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * P.max_unit);
     const float den = group_sum<64>(w * l);
     float num[ND];
 #pragma unroll
@@ -990,17 +1152,29 @@ static bool cache_put_staged(AttnCache* c, const void* k, const void* v, int row
     return true;
 }
 
+enum AttnKernel { ATTN_VALU, ATTN_TILE, ATTN_WIDE };
 struct AttnPlan {
-    bool mfma;  // attn_mfma_kernel (64- or 128-row tiles) instead of attn_split_kernel
+    AttnKernel kernel;
     int rt, row_tiles, splits, keys_per_split, key_end;
 };
 
-// Rows per tile: VALU kernel 4 when a KV head has at most 4 query rows
-// (decode: one row of a 4-head group), else 16; MFMA kernel (16 or more rows
-// per KV head) 64, or 128 from 128 rows on. Keys: enough splits that about
-// 512 blocks run (256 of the 8-wave 128-row blocks, one per CU), each split
-// a whole number of 64-key tiles; with more than one split the blocks write
-// partials (enqueue_attention checks that the workspace holds them).
+// Kernel and rows per tile, for the R = (heads of a group) x rows query rows
+// of a KV head (measured per run, us):
+// - head_dim 256: attn_tile_kernel of 64 rows; at most 4 rows over few keys
+//   (10240 or less over all KV heads, 40 a CU) attn_split_kernel (8 heads of
+//   1000 keys 8.7 against 9.2; 4 of 3000 10.5 against 9.7, 8 of 16000 34.3
+//   against 28.3).
+// - head_dim 64 and 128, R < 16: attn_tile_kernel of 32 rows, weights in 32
+//   bits, 4 waves so that two blocks share a CU (one row of 4-head groups over
+//   3968 keys 8.4; blocks of 16 rows 8.5, of 64 and 8 waves 9.3).
+// - R >= 16: attn_tile_kernel of 64 rows, fp16 weights; 128 rows or more
+//   attn_wide_kernel once a CU's share of the work passes 640 keys of a
+//   64-row tile (8 heads: 512 rows x 2028 keys, 507 keys a CU, 20.6 wide and
+//   19.0 tiles; 512 x 4096, 1024 keys, 25.0 and 26.9).
+// Keys: enough splits that about 512 of the 4-wave blocks run, 256 of the
+// 8-wave ones (one per CU), each split a whole number of tiles; with more than
+// one split the blocks write partials (enqueue_attention checks that the
+// workspace holds them).
 // Overrides for measurement: HM_ATTN_BLOCKS, HM_ATTN_WIDE_BLOCKS (the block
 // counts the key splits aim at).
 static int attn_env(const char* name, int fallback) {
@@ -1011,19 +1185,30 @@ static int attn_env(const char* name, int fallback) {
 static AttnPlan plan_attention(const rk_npu_attention_f16_config& c, int rows, int len, int pos) {
     AttnPlan p;
     const int G = c.query_heads / c.kv_heads, R = G * rows;
-    p.mfma = R >= 16 && (c.head_dim == 64 || c.head_dim == 128);
     static const int env_blocks = attn_env("HM_ATTN_BLOCKS", 512);
     static const int env_wide = attn_env("HM_ATTN_WIDE_BLOCKS", 256);
-    // 128 or more rows per KV head: 8-wave blocks of 128 rows, one per CU
-    // (a K/V tile shared by twice the waves, and the two waves on a SIMD
-    // belong to one block), aiming at HM_ATTN_WIDE_BLOCKS blocks
-    p.rt = p.mfma ? (R >= 128 ? 128 : 64) : (R <= 4 ? 4 : 16);
-    p.row_tiles = (R + p.rt - 1) / p.rt;
     p.key_end = (c.mask_mode == RK_NPU_ATTENTION_F16_CAUSAL) ? std::min(len, pos + rows) : len;
-    const int kt = c.head_dim == 256 ? 32 : ATTN_KT;  // keys per tile of the kernel
+    p.kernel = ATTN_TILE;
+    if (c.head_dim == 256) {
+        p.rt = 64;
+        if (R <= 4 && (long long)c.kv_heads * p.key_end <= 40LL * device_cus()) {
+            p.kernel = ATTN_VALU;
+            p.rt = 4;
+        }
+    } else {
+        p.rt = R < 16 ? 32 : 64;
+        const long long tile_keys = (long long)((R + 63) / 64) * c.kv_heads * p.key_end;
+        if (R > 64 && tile_keys > 640LL * device_cus()) {
+            p.kernel = ATTN_WIDE;
+            p.rt = 128;
+        }
+    }
+    p.row_tiles = (R + p.rt - 1) / p.rt;
+    const int kt = p.kernel == ATTN_VALU ? 32 : ATTN_KT;  // keys per tile of the kernel
     const int tiles = (p.key_end + kt - 1) / kt;
     const int base = p.row_tiles * c.kv_heads;
-    const int target = std::min(std::max(p.rt == 128 ? env_wide : env_blocks, 64), 1024);
+    // (head_dim 256: its partial rows hold 64-row tiles of 256 + base blocks)
+    const int target = std::min(std::max(p.rt >= 64 ? env_wide : env_blocks, 64), c.head_dim == 256 && p.rt == 64 ? 256 : 1024);
     int want = base >= target ? 1 : (target + base - 1) / base;
     want = std::max(1, std::min(std::min(want, tiles), ATTN_MAX_SPLITS));
     const int tiles_per_split = (tiles + want - 1) / want;
@@ -1033,9 +1218,21 @@ static AttnPlan plan_attention(const rk_npu_attention_f16_config& c, int rows, i
     return p;
 }
 
-template <int D, int RT>
-static void launch_attn(const AttnParams& P, const AttnPlan& pl, int kh, hipStream_t s) {
-    hipLaunchKernelGGL((attn_split_kernel<D, RT>), dim3(pl.splits, pl.row_tiles, kh), dim3(256), 0, s, P);
+template <int D>
+static void launch_attn(const AttnParams& P, const AttnPlan& pl, const dim3& grid, hipStream_t s) {
+    if constexpr (D == 256) {
+        if (pl.kernel == ATTN_VALU)
+            hipLaunchKernelGGL((attn_split_kernel<256, 4>), grid, dim3(256), 0, s, P);
+        else
+            hipLaunchKernelGGL((attn_tile_kernel<256, 4, 2, true>), grid, dim3(512), 0, s, P);
+    } else {
+        if (pl.kernel == ATTN_WIDE)
+            hipLaunchKernelGGL(attn_wide_kernel<D>, grid, dim3(64 * ATTN_WIDE_WAVES), 0, s, P);
+        else if (pl.rt == 32)
+            hipLaunchKernelGGL((attn_tile_kernel<D, 2, 2, true>), grid, dim3(256), 0, s, P);
+        else
+            hipLaunchKernelGGL((attn_tile_kernel<D, 4, 2, false>), grid, dim3(512), 0, s, P);
+    }
 }
 
 static int enqueue_attention(AttnWork* w, AttnCache* c, const __half* q, int rows, int pos, void* out, int out_f16,
@@ -1067,31 +1264,15 @@ static int enqueue_attention(AttnWork* w, AttnCache* c, const __half* q, int row
     P.row_tiles = pl.row_tiles;
     P.key_end = pl.key_end;
     P.rows_pad = pl.row_tiles * pl.rt;
+    P.max_unit = pl.kernel == ATTN_VALU ? 1.4426950408889634f : 1.0f;
     const int D = cfg.head_dim;
-#define HM_ATTN(DD)                                                    \
-    if (pl.rt == 4)                                                    \
-        launch_attn<DD, 4>(P, pl, cfg.kv_heads, s);                    \
-    else                                                               \
-        launch_attn<DD, 16>(P, pl, cfg.kv_heads, s);
     const dim3 grid(pl.splits, pl.row_tiles, cfg.kv_heads);
-    if (pl.mfma && D == 64) {
-        if (pl.rt == 128)
-            hipLaunchKernelGGL((attn_mfma_kernel<64, 8>), grid, dim3(512), 0, s, P);
-        else
-            hipLaunchKernelGGL((attn_mfma_kernel<64, 4>), grid, dim3(256), 0, s, P);
-    } else if (pl.mfma && D == 128) {
-        if (pl.rt == 128)
-            hipLaunchKernelGGL((attn_mfma_kernel<128, 8>), grid, dim3(512), 0, s, P);
-        else
-            hipLaunchKernelGGL((attn_mfma_kernel<128, 4>), grid, dim3(256), 0, s, P);
-    } else if (D == 64) {
-        HM_ATTN(64)
-    } else if (D == 128) {
-        HM_ATTN(128)
-    } else {
-        HM_ATTN(256)
-    }
-#undef HM_ATTN
+    if (D == 64)
+        launch_attn<64>(P, pl, grid, s);
+    else if (D == 128)
+        launch_attn<128>(P, pl, grid, s);
+    else
+        launch_attn<256>(P, pl, grid, s);
     if (pl.splits > 1) {
         const int G = cfg.query_heads / cfg.kv_heads;
         // few splits: a wave per row; many: a block per row (measured: 8

@@ -367,3 +367,61 @@ def test_device_append_unaligned_source():
     finally:
         L.rk_npu_attention_f16_cache_free(cache)
         L.rk_npu_attention_f16_workspace_free(ws)
+
+
+@pytest.mark.parametrize("d,qh,kh,rows,length,causal", [
+    # 4 rows over 40 keys per CU and KV head, and one key more (attn_split_kernel / attn_tile_kernel)
+    (256, 32, 8, 1, 1280, True), (256, 32, 8, 1, 1281, True),
+    # 5 rows per KV head; stage and key-group edges (32 and 64 keys); one key
+    (256, 5, 1, 1, 1, True), (256, 8, 1, 4, 31, False), (256, 8, 2, 2, 33, True), (256, 6, 1, 3, 97, True),
+    # 63, 64 and 65 rows per KV head (a full and a ragged row tile), keys over several splits
+    (256, 1, 1, 63, 700, True), (256, 2, 1, 32, 4100, True), (256, 5, 1, 13, 2049, False),
+    # fewer than 16 rows of head_dim 64 / 128 (weights in 32 bits), one key to many splits
+    (128, 4, 4, 1, 1, True), (128, 15, 1, 1, 65, False), (128, 8, 2, 3, 3001, True), (64, 14, 2, 2, 1000, True),
+    # 16 rows on: fp16 weights, 64-row tiles; 128 rows over more than 640 keys a CU (attn_wide_kernel)
+    (128, 4, 1, 4, 130, True), (64, 16, 1, 1, 64, False), (128, 8, 2, 32, 1000, True),
+    (128, 32, 8, 128, 2800, True), (64, 64, 8, 64, 2731, False),
+])
+def test_device_run_plans(d, qh, kh, rows, length, causal):
+    """Every kernel of the attention plan at its edges, f32 and fp16 outputs,
+    q and outputs at 16-byte aligned and 2- (4-)byte aligned addresses.
+
+    With 32-bit weights a score of n = d products carries at most about
+    sqrt(d) 2^-24 of its absolute sum (|s| below 8 here) and the exponential,
+    the sums and the division a few 2^-24 more: 1e-5 of the values' range
+    leaves a factor of 10. fp16 weights: TOL."""
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=64))
+    capacity = -(-length // 32) * 32
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = qh, kh, d, d ** -0.5
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, capacity, capacity
+    cfg.mask_mode = F.RK_NPU_ATTENTION_F16_CAUSAL if causal else F.RK_NPU_ATTENTION_F16_NO_MASK
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    try:
+        g = torch.Generator(device="cuda").manual_seed(length + d)
+        k, v = (torch.randn(kh, length, d, generator=g, device="cuda").half() for _ in range(2))
+        qbuf = torch.randn(qh * rows * d + 1, generator=g, device="cuda").half()
+        stream = torch.cuda.current_stream().cuda_stream
+        npu.check(L.rk_npu_hip_attention_cache_append(cache, k.data_ptr(), v.data_ptr(), length, stream), "append")
+        pos = max(0, length - rows)
+        tol = 1e-5 if d == 256 or qh // kh * rows < 16 else TOL
+        for off in (0, 1):
+            q = qbuf[off:off + qh * rows * d]
+            want = oracle.attention(q.reshape(qh, rows, d).cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(),
+                                    float(np.float32(d ** -0.5)), pos, causal)
+            o32 = torch.empty(qh * rows * d + 1, device="cuda")
+            o16 = torch.empty(qh * rows * d + 1, device="cuda", dtype=torch.float16)
+            for o, half in ((o32, 0), (o16, 1)):
+                npu.check(L.rk_npu_hip_attention_run(ws, cache, q.data_ptr(), rows, pos, o[off:].data_ptr(), half,
+                                                     stream), "run")
+            torch.cuda.synchronize()
+            got32, got16 = (o[off:off + qh * rows * d].reshape(qh, rows, d).cpu().numpy() for o in (o32, o16))
+            close(got32, want, tol)
+            assert np.array_equal(got16, got32.astype(np.float16))
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
