@@ -425,3 +425,51 @@ def test_device_run_plans(d, qh, kh, rows, length, causal):
     finally:
         L.rk_npu_attention_f16_cache_free(cache)
         L.rk_npu_attention_f16_workspace_free(ws)
+
+
+@pytest.mark.parametrize("order", ["null", "side", "null,side", "side,null"])
+def test_host_run_waits_for_device_appends(order):
+    """A host run sees the rows that device appends, still behind other work
+    on their streams when it is called, bring: on the null stream, on another
+    one, on both, and again after new rows."""
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=2048))
+    qh, kh, d, rows = 8, 2, 64, 2
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = qh, kh, d, d ** -0.5
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, 2048, 2048
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    side = torch.cuda.Stream()
+    try:
+        rng = np.random.default_rng(11)
+        busy = torch.randn(4096, 4096, device="cuda")
+        k = rng.standard_normal((kh, 1200, d)).astype(np.float16)
+        v = rng.standard_normal((kh, 1200, d)).astype(np.float16)
+        q = rng.standard_normal((qh, rows, d)).astype(np.float16)
+        kd, vd = (torch.from_numpy(a.view(np.int16)).cuda() for a in (k, v))
+        parts = [(kd[:, i:i + 300].contiguous(), vd[:, i:i + 300].contiguous()) for i in range(0, 1200, 300)]
+        torch.cuda.synchronize()
+        names = order.split(",")
+        for i, (kp, vp) in enumerate(parts):
+            stream = torch.cuda.default_stream() if names[i % len(names)] == "null" else side
+            with torch.cuda.stream(stream):
+                for _ in range(4):
+                    busy = torch.mm(busy, busy).clamp_(-1, 1)
+                npu.check(L.rk_npu_hip_attention_cache_append(cache, kp.data_ptr(), vp.data_ptr(), 300,
+                                                              stream.cuda_stream), "append")
+            if i % 2 == 0 and len(names) > 1:
+                continue  # (the next append, on the other stream, comes first)
+            length = 300 * (i + 1)
+            out = np.empty((qh, rows, d), np.float32)
+            npu.check(L.rk_npu_attention_f16_run(be.ctx, ws, cache, q.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16)),
+                                                 rows, length - rows, out.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
+                                                 None, None), "host run")
+            close(out, oracle.attention(q, k[:, :length], v[:, :length], float(np.float32(d ** -0.5)), length - rows,
+                                        True), 1e-5)
+        torch.cuda.synchronize()
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
