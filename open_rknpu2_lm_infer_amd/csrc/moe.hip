@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "moe_kernels.hpp"
+#include "moe_stream.hpp"
 #include "runtime.hpp"
 
 namespace hm {
@@ -16,6 +17,17 @@ constexpr uint32_t MAGIC_MOE_W = 0x574d4841u;
 constexpr uint32_t MAGIC_MOE_WS = 0x534d4841u;
 constexpr uint32_t BLOB_MAGIC = 0x31584d48u;  // "HMX1"
 constexpr int MOE_BM = 64, MOE_BN = 128;
+// The streamed grouped path (moe_stream.hpp) is taken up to this many slots per
+// expert of the bank: 16-row tiles up to the first, 48-row tiles up to the
+// second. hidden 2048, 128 experts, top 8, intermediate 768, W8 down, us per
+// call, tiled GEMM / 16-row / 48-row tiles: 25 tokens 95 / 65 / 72, 128 (8 slots
+// per expert) 113 / 91 / 98, 256 (16) 121 / 130 / 98, 512 (32) 138 / 214 / 119,
+// 640 (40) 144 / - / 138, 768 (48) 149 / - / 169, where runs past 48 slots make
+// a second pass over their weights.
+constexpr int STREAM_SLOTS_16 = 10, STREAM_SLOTS_48 = 40;
+// Longest intermediate whose codes a block of the 16-row tiles quantizes itself
+// (32 KB of LDS); longer ones are quantized by a launch.
+constexpr int STREAM_AQ_K = 2048;
 
 // One routed expert in device memory: [gate_up payload | gate_up scales |
 // down payload | down scales], each region 256-byte aligned.
@@ -336,6 +348,94 @@ static void launch_slot_gemv(const GemvParams& V, int slots, hipStream_t s) {
         hipLaunchKernelGGL((gemv_kernel<T, 1, BITS, EPI, 8, 2, PREQ, 1, 256, true>), grid, dim3(256), lds, s, V);
 }
 
+// Routing tile of the streamed grouped path, 0: the tiled grouped GEMM. The
+// 48-row tiles only where a block's registers hold its whole share of K: with a
+// reloaded window they lose (hidden 4096, intermediate 1536, 64 experts, 256
+// tokens: 249 us against 211 tiled; 16-row tiles at 30 tokens 171 against 183).
+static int stream_tile(int slots, const MoeBank* b) {
+    if (slots <= STREAM_SLOTS_16 * b->experts) return 16;
+    const bool held = stream_holds(4, b->ggu.K_pad) && stream_holds(b->dn_bits, b->gdn.K_pad);
+    return held && slots <= STREAM_SLOTS_48 * b->experts ? 48 : 0;
+}
+
+// The streamed grouped path up to the contributions: routing and the tokens'
+// codes, gate/up, the middle's codes, down.
+static int enqueue_stream(MoeWork* ws, const MoeBank* b, RouteParams R, int rows, const float* input, hipStream_t s) {
+    const int A = rows * ws->top, bm = stream_tile(A, b);
+    const int tiles = std::min(A, (A + std::min(A, ws->experts) * (bm - 1)) / bm);
+    R.rowmax_count = 0;  // (row maxima leave as one partial per block)
+    TokenQuant Q;
+    Q.x = input;
+    Q.rows = rows;
+    Q.K = ws->h;
+    Q.K_pad = b->ggu.K_pad;
+    Q.vec = ws->h % 16 == 0 && (reinterpret_cast<uintptr_t>(input) & 15) == 0;
+    Q.codes = ws->xws->codes;
+    Q.rowscale = ws->xws->rowscale;
+    Q.rowsum = ws->xws->rowsum;
+    int slot = prof_begin(s, 2, 8, QUANT_MOE, rows, ws->h, 0, "moe_front");
+    launch_moe_front(bm, R, Q, s);
+    prof_end(slot, s);
+
+    MoeStreamParams P{};
+    P.a = ws->xws->codes;
+    P.a_row = b->ggu.K_pad;
+    P.a_plane = 16;
+    P.perm = ws->perm;
+    P.top = ws->top;
+    P.rowscale = ws->xws->rowscale;
+    P.rowsum = ws->xws->rowsum;
+    P.b_tab = b->d_gu;
+    P.s_tab = b->d_gus;
+    P.tiles = ws->tiles;
+    P.counts = ws->counts;
+    P.max_tiles = tiles;
+    P.c = ws->mws->a_f32;  // middle [slot][inter]
+    P.ldc = ws->inter;
+    P.part = ws->gpart;
+    P.N = b->ggu.N;
+    P.K = b->ggu.K;
+    P.K_pad = b->ggu.K_pad;
+    P.half = b->ggu.half;
+    P.tiles_n = (b->ggu.N + 63) / 64;
+    P.staged = 1;
+    slot = prof_begin(s, 3, 4, EPI_SWIGLU_MAX, A, P.K_pad, P.N, "moe_stream<gate_up>");
+    launch_moe_stream(4, EPI_SWIGLU_MAX, bm, false, P, tiles, s);
+    prof_end(slot, s);
+
+    const int parts = P.tiles_n;
+    const bool aq = bm == 16 && b->gdn.K_pad <= STREAM_AQ_K;
+    if (!aq) {
+        const int rc = enqueue_quant(ws->mws, ws->mws->a_f32, DT_F32, ws->inter, A, QUANT_MOE, RowMax{ws->gpart, parts},
+                                     nullptr, s, ws->counts);
+        if (rc != RK_NPU_OK) return rc;
+    }
+    P.a = ws->mws->codes;
+    P.a_row = 16;
+    P.a_plane = (size_t)ws->mws->M_alloc * 16;
+    P.perm = nullptr;
+    P.rowscale = ws->mws->rowscale;
+    P.rowsum = ws->mws->rowsum;
+    P.mid = ws->mws->a_f32;
+    P.part_in = ws->gpart;
+    P.part_count = parts;
+    P.b_tab = b->d_dn;
+    P.s_tab = b->d_dns;
+    P.c = ws->mws->c_f32;  // contributions [slot][h]
+    P.ldc = ws->h;
+    P.part = nullptr;
+    P.N = b->gdn.N;
+    P.K = b->gdn.K;
+    P.K_pad = b->gdn.K_pad;
+    P.half = b->gdn.half;
+    P.tiles_n = (b->gdn.N + 63) / 64;
+    P.staged = ws->h % 4 == 0;
+    slot = prof_begin(s, 3, b->dn_bits, EPI_PLAIN, A, P.K_pad, P.N, "moe_stream<down>");
+    launch_moe_stream(b->dn_bits, EPI_PLAIN, bm, aq, P, tiles, s);
+    prof_end(slot, s);
+    return hipGetLastError() == hipSuccess ? RK_NPU_OK : RK_NPU_ERR_DEVICE;
+}
+
 // Enqueues the whole routed FFN (plus shared expert) for `rows` token rows
 // whose input, ids and routes already sit in device memory.
 static int enqueue_moe(MoeWork* ws, const MoeBank* b, int rows, const float* input, const int* ids,
@@ -354,19 +454,21 @@ static int enqueue_moe(MoeWork* ws, const MoeBank* b, int rows, const float* inp
     // quantization launch); otherwise the rows are quantized first.
     const bool slot_quant = slot_gemv && (ws->h % 16) == 0 && (reinterpret_cast<uintptr_t>(input) & 15) == 0 &&
                             (b->ggu.K_pad / 16) <= 256 * GEMV_XMAX;
+    // More slots, few per expert: the weights are the bound, and the streamed
+    // kernels read them at the rate of a copy.
+    const bool stream = !slot_gemv && stream_tile(A, b) != 0;
     // Many slots: after routing, the tokens' rows are quantized straight into
     // slot order (slot s holds token perm[s] / top), so the grouped GEMM's A
     // loads are contiguous rows; one launch for what was a token quantization
     // and a gather of its codes (measured at 4096 slots: gate/up 69 -> 57 us
     // with contiguous rows). Few slots: the tokens are quantized once and the
     // GEMM gathers rows itself.
-    const bool slot_order = !slot_gemv && A >= 256;
+    const bool slot_order = !slot_gemv && !stream && A >= 256;
     int rc = RK_NPU_OK;
-    if (!slot_quant && !slot_order) {
+    if (!slot_quant && !slot_order && !stream) {
         rc = enqueue_quant(ws->xws, input, DT_F32, ws->h, rows, QUANT_MOE, RowMax{nullptr, 0}, nullptr, s);
         if (rc != RK_NPU_OK) return rc;
     }
-    if (!slot_gemv) {
     RouteParams R;
     R.ids = ids;
     R.routes = routes;
@@ -380,7 +482,11 @@ static int enqueue_moe(MoeWork* ws, const MoeBank* b, int rows, const float* inp
     R.rowmax_mid = ws->mws->rowmax;
     R.rowmax_count = A;
     R.error = ws->error;
-    hipLaunchKernelGGL(moe_route_kernel<MOE_BM>, dim3(1), dim3(1024), 0, s, R);
+    if (stream) {
+        rc = enqueue_stream(ws, b, R, rows, input, s);
+        if (rc != RK_NPU_OK) return rc;
+    } else if (!slot_gemv) {
+        hipLaunchKernelGGL(moe_route_kernel<MOE_BM>, dim3(1), dim3(1024), 0, s, R);
     }
 
     if (slot_gemv) {
@@ -464,7 +570,7 @@ static int enqueue_moe(MoeWork* ws, const MoeBank* b, int rows, const float* inp
         if (rc != RK_NPU_OK) return rc;
     }
 
-    if (!slot_gemv) {
+    if (!slot_gemv && !stream) {
     MoeGemmParams G;
     G.a = slot_order ? ws->gcodes : ws->xws->codes;
     G.a_alloc = slot_order ? ws->g_alloc : ws->xws->M_alloc;

@@ -31,7 +31,7 @@ struct RouteParams {
 };
 
 template <int BM>
-__global__ __launch_bounds__(1024) void moe_route_kernel(RouteParams P) {
+__device__ __forceinline__ void moe_route_block(const RouteParams& P) {
     __shared__ int cnt[MOE_MAX_EXPERTS];
     __shared__ int fill[MOE_MAX_EXPERTS];
     __shared__ int off[MOE_MAX_EXPERTS];
@@ -138,6 +138,11 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(RouteParams P) {
             P.tiles[toff[e] + t] = make_int4(e, b, min(off[e] + cnt[e], b + BM), 0);
         }
     }
+}
+
+template <int BM>
+__global__ __launch_bounds__(1024) void moe_route_kernel(RouteParams P) {
+    moe_route_block<BM>(P);
 }
 
 // ---------------------------------------------------------------------------
