@@ -1938,7 +1938,7 @@ def profile_attention(stats_csv, attn_json, pmc1_csv, pmc2_csv):
            "      <pmc1>/<host>/<pid>_run_counter_collection.csv <pmc2>/<host>/<pid>_run_counter_collection.csv", "",
            "Workload (bench.py run_attention): one rk_npu_hip_attention_run per layer cache; decode = 1 query row at",
            "the last position (attn_split_kernel + attn_combine_kernel), prefill = 128 query rows ending at the last",
-           "position, causal (attn_mfma_kernel + attn_combine_rows_kernel); eager steps and graph replays both in",
+           "position, causal (attn_wide_kernel + attn_combine_rows_kernel); eager steps and graph replays both in",
            "the table.", ""]
     out += _stats_table(stats_csv)
     r1, r2 = _counters(pmc1_csv), _counters(pmc2_csv)
