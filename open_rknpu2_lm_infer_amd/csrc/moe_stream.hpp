@@ -109,8 +109,8 @@ __global__ __launch_bounds__(FRONT_THREADS) void moe_front_kernel(RouteParams R,
 // 768, 128 experts, top 8, us, tiled -> streamed:
 //                        25 tokens (161 MB each)    512 tokens (201 MB each)
 //   route + token codes     9.8 -> 4.6                 17.7 -> 6.2
-//   gate/up W4             44.7 -> 29.4 (5.5 TB/s)     62.4 \ 114.8 -> 98 together
-//   down W8                33.9 -> 28.0 (5.8 TB/s)     52.4 / (and 46 MB written)
+//   gate/up W4             44.7 -> 29.4 (5.5 TB/s)     62.4 -> 59.2 (3.4 TB/s)
+//   down W8                33.9 -> 28.0 (5.8 TB/s)     52.4 -> 44.2 (4.6 TB/s, and 34 MB written)
 //   middle's codes          5.0 -> in down              7.3 -> 5.7
 //   whole call             89.0 -> 64.0               135.3 -> 117.2
 // 48 rows and two code steps in flight let three blocks share a CU; 64 rows
