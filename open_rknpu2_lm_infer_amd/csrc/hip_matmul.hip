@@ -471,7 +471,9 @@ static bool plan_skinny(int rows, const Geometry& g, int epi, bool gemv, SkinnyP
     p.row_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : 8;
     const int groups = (rows + 16 * p.row_tiles - 1) / (16 * p.row_tiles);
     p.col_tiles = epi != EPI_PLAIN || g.N_pad / 16 * groups > cus ? 2 : 1;
-    p.blocks_n = g.N_pad / (16 * p.col_tiles);
+    // (SwiGLU: a block per pair of a gate and an up tile and none for padding
+    // columns, as every block's row maxima are read; N is a multiple of 64)
+    p.blocks_n = epi != EPI_PLAIN ? g.N / 32 : g.N_pad / (16 * p.col_tiles);
     if (forced > 0) return true;
     if (gemv && (rows <= 2 || (rows <= 4 && g.bits == 8))) return false;
     if (rows <= 64) return true;

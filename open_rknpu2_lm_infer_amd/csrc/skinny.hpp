@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64 * NWV) void skinny_kernel(SkinnyParams S) {
     const int b = blockIdx.x;
     const int col0 = EPI == EPI_PLAIN ? b * 16 * CT : (b >> 1) * 64 + (b & 1) * 16;
     constexpr int CSTEP = EPI == EPI_PLAIN ? 16 : 32;
-    if (col0 >= P.N) return;  // (a tile of padding columns only)
+    if (col0 >= P.N) return;  // (tiles of padding columns only; none of SwiGLU's)
     const int row0 = blockIdx.y * (16 * RT);
 
     const int planes = P.K_pad / (BITS == 8 ? 16 : 32);

@@ -161,6 +161,28 @@ def test_moe_with_shared_w8_expert(rows, top, qw, fuse):
     assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("dn_bits", [4, 8])
+def test_shared_expert_after_a_one_token_call(dn_bits):
+    """A shared expert whose gate_up width is off 256 (padding columns): a call of
+    one much larger token leaves its row maxima in the workspace that a later
+    call of 16 tokens uses; each call is requantized by its own rows' maxima."""
+    h, inter, experts, top = 512, 160, 8, 2
+    backend = npu.Backend(npu.ModelOptions(chunk=16))
+    gate, down = moe_bank(h, inter, experts, dn_bits, f"moeshp{dn_bits}")
+    sg = npu.QuantMatrix(8, h, 2 * inter, *R.weights(4, "shp-gu", 8, h, 2 * inter))
+    sd = npu.QuantMatrix(8, inter, h, *R.weights(4, "shp-dn", 8, inter, h))
+    moe = backend.load_moe_with_shared(gate, down, top, (sg, sd))
+    for rows, scale in ((1, 100.0), (16, 1.0), (2, 100.0), (5, 1.0)):
+        x = R.activations(4, f"moeshp-x{rows}", rows, h) * np.float32(scale)
+        ids, w = routed(rows, experts, top, f"moeshp-r{rows}")
+        out = np.zeros((rows, h), np.float32)
+        print(f"shared expert, W{dn_bits} down, {rows} rows", flush=True)
+        moe.run(x, ids, w, out, rows)
+        ref = oracle.moe([(g.codes, g.scales) for g in gate], [(d.codes, d.scales) for d in down], x, ids, w,
+                         shared=((sg.codes, sg.scales), (sd.codes, sd.scales)))
+        assert np.array_equal(out, ref)
+
+
 def test_moe_rejects_out_of_range_ids():
     backend = npu.Backend(npu.ModelOptions(chunk=4))
     gate, down = moe_bank(64, 32, 4, 4, "moebad")

@@ -113,3 +113,26 @@ def test_skinny_static_entry(ctx, bits, rows):
                                                        F.RK_NPU_HIP_F32, rows, epi, D.current_stream()), "static")
         torch.cuda.synchronize()
         assert np.array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("f", [1056, 2080])
+@pytest.mark.parametrize("gu_bits,dn_bits", [(4, 4), (8, 8)])
+def test_ffn_row_maxima_after_a_gemv_call(ctx, gu_bits, dn_bits, f):
+    """One workspace pair for every row count, its gate_up width off 256
+    (padding columns): after a call of a few much larger rows on the GEMV, which
+    leaves its maxima in the same buffer, later calls requantize the middle by
+    their own rows' maxima only."""
+    h, most = 512, 64
+    gc, gs = R.weights(25, f"skag{gu_bits}-{f}", gu_bits, h, 2 * f)
+    dc, ds = R.weights(25, f"skad{dn_bits}-{f}", dn_bits, f, h)
+    gu, dn = ctx.weights(gu_bits, dev(gc), dev(gs)), ctx.weights(dn_bits, dev(dc), dev(ds))
+    gws, dws = ctx.workspace(gu_bits, most, h, 2 * f), ctx.workspace(dn_bits, most, f, h)
+    for first in (1, 2, 4):
+        for rows in (3, 8, 16, 64):
+            for n, scale in ((first, 100.0), (rows, 1.0)):
+                print(f"W{gu_bits}/W{dn_bits} f={f} {n} rows after {first}", flush=True)
+                x = R.activations(25, f"ska-x{n}-{first}-{rows}", n, h) * np.float32(scale)
+                y = torch.empty(n, h, dtype=torch.float32, device="cuda")
+                D.ffn(ctx, gu, dn, dev(x), y, n, gws=gws, dws=dws)
+                torch.cuda.synchronize()
+                assert np.array_equal(y.cpu().numpy(), oracle.ffn(gc, gs, dc, ds, x))
