@@ -134,7 +134,9 @@ int rk_npu_attention_f16_run_half(rk_npu_ctx* ctx, rk_npu_attention_f16_workspac
 /* ---- device-resident entry points (no reference counterpart) ------------
  * For callers whose K/V/Q/output already live in HBM (same layouts as the
  * host calls), on the caller's HIP stream (NULL: the null stream); nothing
- * is synchronized. out_f16 selects fp16 output. */
+ * is synchronized. out_f16 selects fp16 output. Appended rows in the cache's
+ * own GPU's memory, 16-byte aligned, are read by a kernel; others go through
+ * hipMemcpy2DAsync. */
 int rk_npu_hip_attention_cache_append(rk_npu_attention_f16_cache* cache, const void* k_dev, const void* v_dev,
                                       int32_t rows, void* stream);
 int rk_npu_hip_attention_run(rk_npu_attention_f16_workspace* workspace, rk_npu_attention_f16_cache* cache,

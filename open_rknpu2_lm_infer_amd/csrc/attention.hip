@@ -1144,6 +1144,19 @@ __global__ __launch_bounds__(256) void attn_append_kernel(const v4u* __restrict_
     for (int i = blockIdx.x * 256 + threadIdx.x; i < pieces; i += gridDim.x * 256) dst[i] = src[i];
 }
 
+// Whether a kernel on `device` may read caller memory at p: that GPU's own.
+// Another GPU's (readable only where peer access is on), managed and host
+// memory (pageable memory faults a kernel) keep the copies, which the runtime
+// checks and stages.
+static bool kernel_readable(const void* p, int device) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
 // Launches it for `rows` rows whose K and V lie at 16-byte aligned device (or
 // mapped host) addresses; the caller advances the length.
 static void enqueue_append(AttnCache* c, const void* k, const void* v, int rows, hipStream_t s) {
@@ -1593,7 +1606,8 @@ int rk_npu_hip_attention_cache_append(rk_npu_attention_f16_cache* cache, const v
     if ((long)c->length + rows > c->capacity) return RK_NPU_ERR_PARAM;  // (reserve first: no allocation here)
     if (hipSetDevice(device_of(c->domain)) != hipSuccess) return RK_NPU_ERR_DEVICE;
     int rc;
-    if (((reinterpret_cast<uintptr_t>(k_dev) | reinterpret_cast<uintptr_t>(v_dev)) & 15) == 0) {
+    if (((reinterpret_cast<uintptr_t>(k_dev) | reinterpret_cast<uintptr_t>(v_dev)) & 15) == 0 &&
+        kernel_readable(k_dev, device_of(c->domain)) && kernel_readable(v_dev, device_of(c->domain))) {
         enqueue_append(c, k_dev, v_dev, rows, static_cast<hipStream_t>(stream));
         rc = hipGetLastError() == hipSuccess ? RK_NPU_OK : RK_NPU_ERR_DEVICE;
         if (rc == RK_NPU_OK) c->length += rows;

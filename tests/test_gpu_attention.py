@@ -473,3 +473,65 @@ def test_host_run_waits_for_device_appends(order):
     finally:
         L.rk_npu_attention_f16_cache_free(cache)
         L.rk_npu_attention_f16_workspace_free(ws)
+
+
+def test_device_append_reads_only_its_gpus_memory_by_a_kernel():
+    """Aligned rows in device memory are appended by one kernel; every other
+    source (host memory here, as another GPU's would) by the two 2-D copies, whose
+    checks and staging it needs. Shown by the nodes that a capture records, and by
+    the rows that an append from host memory leaves."""
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=64))
+    qh, kh, d, rows = 4, 2, 64, 9
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = qh, kh, d, d ** -0.5
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, 64, 64
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    side = torch.cuda.Stream()
+    stream = ctypes.c_void_p(side.cuda_stream)
+    host = [torch.randn(kh, rows, d, generator=torch.Generator().manual_seed(i)).half().pin_memory() for i in (1, 2)]
+    device = [t.cuda() for t in host]
+    q = torch.randn(qh, rows, d, device="cuda").half()
+
+    def nodes(k, v):
+        graph, count = ctypes.c_void_p(), ctypes.c_size_t()
+        npu.check(L.rk_npu_attention_f16_cache_truncate(cache, 0), "truncate")
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # (relaxed)
+        rc = L.rk_npu_hip_attention_cache_append(cache, k.data_ptr(), v.data_ptr(), rows, stream)
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0 and rc == 0
+        try:
+            assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+            handles = (ctypes.c_void_p * count.value)()
+            assert hip.hipGraphGetNodes(graph, handles, ctypes.byref(count)) == 0
+            kinds = []
+            for node in handles:
+                kind = ctypes.c_int()
+                assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+                kinds.append(kind.value)
+            return kinds
+        finally:
+            assert hip.hipGraphDestroy(graph) == 0
+
+    kernel, copy = 0, 1  # (hipGraphNodeTypeKernel, hipGraphNodeTypeMemcpy)
+    try:
+        torch.cuda.synchronize()
+        assert nodes(*device) == [kernel]
+        assert nodes(*host) == [copy, copy]
+        assert nodes(device[0], host[1]) == [copy, copy]
+        outs = []
+        for k, v in (device, host):
+            out = torch.empty(qh, rows, d, device="cuda")
+            npu.check(L.rk_npu_attention_f16_cache_truncate(cache, 0), "truncate")
+            npu.check(L.rk_npu_hip_attention_cache_append(cache, k.data_ptr(), v.data_ptr(), rows, stream), "append")
+            npu.check(L.rk_npu_hip_attention_run(ws, cache, q.data_ptr(), rows, 0, out.data_ptr(), 0, stream), "run")
+            torch.cuda.synchronize()
+            outs.append(out.cpu())
+        assert torch.equal(*outs)
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
