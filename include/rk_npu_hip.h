@@ -143,7 +143,8 @@ int rk_npu_hip_inject_alloc_failures(int count);
  *   HM_GEMM_VARIANT  -1 by shape; 0..5 forces the 256x256, 256x128, 128x128,
  *                    64x128, 32x128 or 192x256 GEMM tile
  *   HM_SPLITS        0 by shape; n > 0 forces n K pieces per GEMM tile
- *   HM_FORCE_GEMM    1: rows <= 8 take the MFMA GEMM instead of the GEMV
+ *   HM_FORCE_GEMM    1: rows <= 8 take the tiled MFMA GEMM instead of the GEMV
+ *                    or the kernel of HM_SKINNY (which at 1 comes first)
  *   HM_SKINNY        -1 by shape; 0 never, 1 always (up to 256 rows): the
  *                    kernel that streams the weights into matrix-core
  *                    operands instead of the GEMV or the tiled GEMM (not when

@@ -460,13 +460,15 @@ constexpr int SKINNY_MAX_ROWS = 256;
 // - one column tile per block while the blocks fit one per CU, else two (o of
 //   16 rows W4 one 7.5, two 8.1; qkv 7.8 and 7.5, of 128 rows 14.5 and 12.2).
 // HM_SKINNY: 0 never, 1 always up to SKINNY_MAX_ROWS rows. A forced GEMM tile
-// or split (HM_GEMM_VARIANT, HM_SPLITS) keeps the tiled GEMM.
+// or split (HM_GEMM_VARIANT, HM_SPLITS) keeps the tiled GEMM, as does
+// HM_FORCE_GEMM for its rows unless HM_SKINNY is 1.
 constexpr size_t skinny_code_bytes = (size_t)576 << 10;
 
 static bool plan_skinny(int rows, const Geometry& g, int epi, bool gemv, SkinnyPlan& p) {
     const int forced = switch_value(SW_SKINNY);
     if (forced == 0 || rows > SKINNY_MAX_ROWS || switch_value(SW_GEMM_VARIANT) >= 0 || switch_value(SW_SPLITS) > 0)
         return false;
+    if (forced < 0 && rows <= 8 && switch_value(SW_FORCE_GEMM) != 0) return false;
     const int cus = device_cus();
     p.row_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : 8;
     const int groups = (rows + 16 * p.row_tiles - 1) / (16 * p.row_tiles);

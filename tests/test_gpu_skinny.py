@@ -136,3 +136,22 @@ def test_ffn_row_maxima_after_a_gemv_call(ctx, gu_bits, dn_bits, f):
                 D.ffn(ctx, gu, dn, dev(x), y, n, gws=gws, dws=dws)
                 torch.cuda.synchronize()
                 assert np.array_equal(y.cpu().numpy(), oracle.ffn(gc, gs, dc, ds, x))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("rows", [1, 2, 4, 8, 16])
+def test_forced_gemm_is_the_tiled_one(ctx, bits, rows):
+    """HM_FORCE_GEMM sends rows <= 8 to the tiled GEMM instead of the GEMV (more
+    rows take what they take without it); HM_SKINNY=1 comes before it."""
+    k, n = 512, 320
+    codes, scales = R.weights(26, f"skfg{bits}", bits, k, n)
+    w = ctx.weights(bits, dev(codes), dev(scales))
+    x = R.activations(26, f"skfg-x{rows}", rows, k)
+    ws = ctx.workspace(bits, 16, k, n)
+    for skinny, kernel in ((-1, "gemm<" if rows <= 8 else "skinny<"), (1, "skinny<")):
+        y = torch.empty(rows, n, device="cuda")
+        with D.plan_switch("HM_FORCE_GEMM", 1), D.plan_switch("HM_SKINNY", skinny), D.KernelProfile(16) as p:
+            D.linear(ctx, w, dev(x), y, rows, ws=ws)
+            torch.cuda.synchronize()
+        assert [s["name"].startswith(kernel) for s in p.stats if s["kind"] < 2] == [True], p.stats
+        assert np.array_equal(y.cpu().numpy(), oracle.linear(codes, scales, x))
