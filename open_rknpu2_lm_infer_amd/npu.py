@@ -79,19 +79,34 @@ def _ptr(a: np.ndarray, t):
 
 class _Handle:
     """Owning native pointer. `keep` holds whatever must outlive it (the
-    context and domain), so finalization order never frees a domain before
-    the weights and workspaces allocated in it."""
+    context and domain). Reference counts free a domain after the weights and
+    workspaces allocated in it; in a garbage cycle the collector finalizes in any
+    order, so a handle that others still depend on is freed by the last of them."""
 
     def __init__(self, raw, free, name: str, keep=None):
         ensure(bool(raw), f"cannot allocate {name}")
         self.raw = raw
         self._free = free
         self._keep = keep
+        self._dependents = set()
+        self._closing = False
+        parent = getattr(keep, "domain", keep)
+        self._parent = parent if isinstance(parent, _Handle) else None
+        if self._parent is not None:
+            self._parent._dependents.add(id(self))
 
     def close(self):
-        if self.raw:
-            self._free(self.raw)
-            self.raw = None
+        if not self.raw:
+            return
+        if self._dependents:
+            self._closing = True
+            return
+        self._free(self.raw)
+        self.raw = None
+        if self._parent is not None:
+            self._parent._dependents.discard(id(self))
+            if self._parent._closing:
+                self._parent.close()
 
     def __del__(self):
         try:

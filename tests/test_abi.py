@@ -315,3 +315,29 @@ def test_non_hot_entry_points_report_unsupported_without_a_device():
     for name in ("rk_npu_mm_plan_free", "rk_npu_mm_workspace_free", "rk_npu_mla_f16_cache_free",
                  "rk_npu_gdn_workspace_free", "rk_npu_mm_gelu_free", "rk_npu_mm_tuned_weights_free"):
         getattr(L, name)(None)
+
+
+@pytest.mark.parametrize("in_cycle", [False, True])
+def test_handles_free_in_dependency_order(in_cycle):
+    """A context outlives its domain and a domain what is allocated in it, also
+    when all of them die as one garbage cycle (which the collector finalizes in
+    the order they were made)."""
+    import gc
+    freed = []
+
+    class Owner:
+        pass
+
+    gc.collect()
+    owner = Owner()
+    owner.ctx = npu._Handle(1, lambda raw: freed.append("ctx"), "context")
+    owner.domain = npu._Handle(2, lambda raw: freed.append("domain"), "domain", keep=owner.ctx)
+    owner.parts = [npu._Handle(3 + i, lambda raw, i=i: freed.append(f"part{i}"), "part", keep=owner) for i in range(2)]
+    if in_cycle:
+        owner.me = owner
+    else:
+        parts, owner.parts = owner.parts, None  # (they hold their owner)
+        del parts
+    del owner
+    gc.collect()
+    assert sorted(freed[:2]) == ["part0", "part1"] and freed[2:] == ["domain", "ctx"], freed
