@@ -90,6 +90,27 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// An output that came out NaN, of query row qrow (within its head) of KV head g
+// with weights' sum l. An infinity among the values it sees makes it that
+// infinity; the kernels' sums hold NaN then wherever a weight of 0 met it: the
+// remainder of a weight split in two, a key past the split, a split's weight.
+// NaN stays where a weight or a value is NaN or the infinities have both signs.
+__device__ __forceinline__ float nan_output(const AttnParams& P, int g, int qrow, int D, int dim, float l) {
+    const __half* v = P.v + (size_t)g * P.cap * D + dim;
+    const int keys = l == l ? (P.causal ? min(P.len, P.pos + qrow + 1) : P.len) : 0;
+    bool up = false, down = false, nan = false;
+    for (int j = 0; j < keys && !nan; j += 16) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {  // (one memory round trip for 16 keys)
+            const unsigned b = reinterpret_cast<const unsigned short*>(v)[(size_t)min(j + u, keys - 1) * D];
+            up |= b == 0x7C00u;
+            down |= b == 0xFC00u;
+            nan |= (b & 0x7FFFu) > 0x7C00u;
+        }
+    }
+    return nan || up == down ? NAN : up ? INFINITY : -INFINITY;
+}
+
 // Block: 256 threads; RT query rows (4: 64 threads per row), head_dim 256.
 // Thread (row, sub) scores key sub of each tile and owns output dims
 // [sub*DPT, sub*DPT + DPT) of its row. K/V tiles of 32 keys go through LDS;
@@ -535,7 +556,12 @@ __global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnPar
 // row's largest weight. Against 64 bits the outputs are nearer than the VALU
 // kernels' whose place this took (f32 weights, v_dot2 scores): 128 rows of 8-head
 // groups of 256 over 2048 keys 3.0e-7 (5.8e-7), one row of 128 over 16000
-// 2.9e-7 (4.4e-7). Calls that had fp16 weights keep them (SPLIT = false).
+// 2.9e-7 (4.4e-7). Over 147 shapes of one to 800 rows per KV head, 65 to 16000
+// keys and every head_dim, each at three spreads of the scores, the error is
+// 0.59 times theirs (geometric mean; largest at normal q and k 4.6e-7, theirs
+// 1.4e-6). An infinite value leaves NaN with a remainder of 0 or below;
+// nan_output puts that right. Calls that had fp16 weights keep them (SPLIT =
+// false).
 //
 // Measured per run with its combine, us, the kernels before -> this (one row =
 // one query row, so 4 or 8 rows per KV head):
@@ -593,7 +619,7 @@ __global__ __launch_bounds__(64 * WR * WK) void attn_tile_kernel(AttnParams P) {
     auto swv = [](int r) { return D >= 128 ? 2 * (r & 7) : 2 * ((r >> 1) & 3); };
 
     auto issue = [&](int kb, v4u (&kr)[PT], v4u (&vr)[PT]) {
-        const int last = k1 - 1 - kb;  // (keys past the split read its last key: finite data, masked)
+        const int last = k1 - 1 - kb;  // (keys past the split read its last key, masked)
 #pragma unroll
         for (int t = 0; t < PT; ++t) {
             const int i = t * NT + tid;
@@ -757,9 +783,22 @@ __global__ __launch_bounds__(64 * WR * WK) void attn_tile_kernel(AttnParams P) {
     if (P.splits == 1) {
         const float inv = 1.0f / l;
         const size_t o0 = ((size_t)(g * G + rr / P.m) * P.m + rr % P.m) * D + 4 * hi;
+        float sum = 0.0f;
 #pragma unroll
         for (int n = 0; n < NB; ++n) {
-            const f4 y = o[n] * inv;
+            o[n] *= inv;
+            sum += (o[n][0] + o[n][1]) + (o[n][2] + o[n][3]);
+        }
+        if (__builtin_expect(sum != sum, 0)) {
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (o[n][r] != o[n][r]) o[n][r] = nan_output(P, g, rr % P.m, D, 16 * n + 4 * hi + r, l);
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const f4 y = o[n];
             if (P.out_f16) {
                 const unsigned short b0 = __half_as_ushort(__float2half_rn(y[0]));
                 const unsigned short b1 = __half_as_ushort(__float2half_rn(y[1]));
@@ -856,7 +895,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams P) {
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
             const int dd = lane + 64 * d;
-            const float y = ((sums[0][dd] + sums[1][dd]) + (sums[2][dd] + sums[3][dd])) * inv;
+            float y = ((sums[0][dd] + sums[1][dd]) + (sums[2][dd] + sums[3][dd])) * inv;
+            if (__builtin_expect(y != y, 0)) y = nan_output(P, g, qr, D, dd, inv);
             if (P.out_f16)
                 static_cast<__half*>(P.out)[o + 64 * d] = __float2half_rn(y);
             else
@@ -918,7 +958,8 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(AttnParams P) {
     const size_t o = ((size_t)h * P.m + qr) * D + lane;
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
-        const float y = num[d] * inv;
+        float y = num[d] * inv;
+        if (__builtin_expect(y != y, 0)) y = nan_output(P, g, qr, D, lane + 64 * d, den);
         if (P.out_f16)
             static_cast<__half*>(P.out)[o + 64 * d] = __float2half_rn(y);
         else

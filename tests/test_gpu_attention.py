@@ -535,3 +535,45 @@ def test_device_append_reads_only_its_gpus_memory_by_a_kernel():
     finally:
         L.rk_npu_attention_f16_cache_free(cache)
         L.rk_npu_attention_f16_workspace_free(ws)
+
+
+@pytest.mark.parametrize("where", [0, 0.4, 1])
+@pytest.mark.parametrize("d,qh,kh,rows,length", [(256, 16, 2, 16, 1000), (256, 16, 2, 1, 3000), (256, 8, 1, 1, 1),
+                                                 (128, 32, 8, 1, 1000), (128, 32, 8, 16, 1000), (128, 8, 1, 12, 16001),
+                                                 (64, 8, 8, 2, 777), (64, 15, 1, 1, 64)])
+def test_infinite_values(d, qh, kh, rows, length, where):
+    """An infinity in V at the first key, one inside and the last (of a split
+    that ends inside a tile) gives infinities of its sign in its column and moves
+    no other: a weight's two fp16 parts and the keys past a split are no NaN."""
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=64))
+    capacity = -(-length // 32) * 32
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = qh, kh, d, d ** -0.5
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, capacity, capacity
+    cfg.mask_mode = F.RK_NPU_ATTENTION_F16_NO_MASK
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    try:
+        g = torch.Generator(device="cuda").manual_seed(length + d)
+        k, v = (torch.randn(kh, length, d, generator=g, device="cuda").half() for _ in range(2))
+        q = torch.randn(qh, rows, d, generator=g, device="cuda").half()
+        stream = torch.cuda.current_stream().cuda_stream
+        key, outs = min(int(where * length), length - 1), []
+        for value in (0.0, float("inf"), float("-inf")):
+            v[:, key, 3] = value
+            out = torch.empty(qh, rows, d, device="cuda")
+            npu.check(L.rk_npu_attention_f16_cache_truncate(cache, 0), "truncate")
+            npu.check(L.rk_npu_hip_attention_cache_append(cache, k.data_ptr(), v.data_ptr(), length, stream), "append")
+            npu.check(L.rk_npu_hip_attention_run(ws, cache, q.data_ptr(), rows, 0, out.data_ptr(), 0, stream), "run")
+            torch.cuda.synchronize()
+            outs.append(out.cpu())
+            if value:
+                assert torch.all(out[:, :, 3] == value)
+                keep = torch.arange(d) != 3
+                assert torch.equal(outs[-1][:, :, keep], outs[0][:, :, keep])
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
