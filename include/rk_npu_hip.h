@@ -203,9 +203,9 @@ int rk_npu_hip_profile_read(rk_npu_hip_kernel_stat* stats, int capacity, int* co
 
 /* Launch plan of a linear of this shape, for diagnostics: kind 0 = GEMV, 1 =
  * tiled MFMA GEMM; tile sizes and K splits. It is the plan that sizes the
- * workspace and that HM_SKINNY=0 launches: by default most calls of 3 to 64
- * rows, and of up to 256 where few column tiles share the codes, run on the
- * streaming kernel instead (HM_SKINNY). */
+ * workspace and that HM_SKINNY=0 launches: by default calls of 3 to 256 rows
+ * run on the streaming kernel instead (HM_SKINNY) where it is the faster one,
+ * mostly those whose column tiles give a CU few blocks. */
 typedef struct rk_npu_hip_plan {
     int32_t kind;
     int32_t block_m;

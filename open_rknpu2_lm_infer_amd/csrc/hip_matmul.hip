@@ -445,42 +445,75 @@ Plan plan_linear(int rows, const Geometry& g) {
 // --- few rows: skinny_kernel ---------------------------------------------------
 constexpr int SKINNY_MAX_ROWS = 256;
 
-// Whether a call of `rows` rows runs on skinny_kernel, and how. Lines drawn by
-// measurement (per call with the quantization launch, us, other path -> this):
-// - 1 or 2 rows stay with the GEMV, which needs no quantization launch (qkv
-//   2560x6144 W4 of 2 rows 6.3 -> 7.3). 3 or 4 rows of W4 come here (gate_up
-//   2560x19456 13.4 -> 11.6, down 9728x2560 11.2 -> 10.8, qkv 8.0 -> 7.3), of
-//   W8 they stay (up 2560x9728 9.8 -> 11.1). 5 to 8 rows come here (W4 qkv
-//   9.3 -> 7.4, gate_up 16.9 -> 11.7; W8 o 9.8 -> 8.5, gate_up 19.2 -> 17.2).
-// - up to 64 rows every measured shape gains (skinny.hpp).
-// - above, up to 256, the codes a CU reads decide: blocks per CU, rounded up,
-//   times the block's rows, times K. qkv of 128 rows (320 KB) 15.2 -> 12.2 and
-//   o 4096x2560 of 128 (512 KB) 19.7 -> 13.0, of 256 (512 KB) 20.5 -> 15.0;
-//   qkv of 256 (640 KB) 16.1 -> 19.2, up 2560x9728 of 128 (640 KB) 16.4 -> 18.7.
-// - one column tile per block while the blocks fit one per CU, else two (o of
-//   16 rows W4 one 7.5, two 8.1; qkv 7.8 and 7.5, of 128 rows 14.5 and 12.2).
-// HM_SKINNY: 0 never, 1 always up to SKINNY_MAX_ROWS rows. A forced GEMM tile
-// or split (HM_GEMM_VARIANT, HM_SPLITS) keeps the tiled GEMM, as does
-// HM_FORCE_GEMM for its rows unless HM_SKINNY is 1.
-constexpr size_t skinny_code_bytes = (size_t)576 << 10;
+// Whether skinny_kernel is the faster path for a call of `rows` rows that it
+// would run as plan p. Its time goes with the blocks a CU runs (per_cu, rounded
+// up: each reads the rows' codes for all of K and merges its waves' sums), the
+// other path's with K (the tiled GEMM: a stage per 64) and the output. The lines
+// are those of a sweep of both paths over 105 products, K 512 to 9728 by N 512 to
+// 19456, 576x1536 to 8192x28672 and 1024 and 2560x151936, plain and SwiGLU, W4
+// and W8, 17 row counts from 3 to 256 (distinct weights in a graph, both paths with
+// their quantization launch). Time on skinny_kernel over the other's:
+//   plain, against the tiled GEMM   W4                      W8
+//    to 16 rows, 1 / 2 / 3 a CU     .29-.79 .50-.87 .66-.99 .33-.87 .72-1.07 .89-1.23
+//    to 32                          .34-.83 .64-.94 .81-1.09 .41-.92 .80-1.17 .97-1.39
+//    to 64                          .48-1.0 .79-1.2 .96-1.35 .53-1.1 .96-1.45 1.2-1.8
+//    to 256                         .61-1.3 1.1-1.7 1.3-1.9  .67-1.5 1.2-1.7  1.1-2.2
+//   SwiGLU: to 64 rows W4 .42-.73 up to 3 a CU, .68-.95 at 4 (8192x28672); W8
+//    .48-1.01, 1.00-1.15 at 4; to 256 rows W4 .61-.99 up to 2, .83-1.58 beyond, W8
+//    .73-1.03 at 1, .96-1.58 beyond
+// and a wide range within a cell is K: the tiled GEMM splits K from 8192 on, and
+// below about 1500 it has few stages. Against the GEMV (no quantization launch
+// up to 2 rows): W4 of 5 to 8 rows .50-.93, of 3 and 4 .61-1.0 except long K in
+// blocks that leave the last round part empty (9728x512 1.2, 6144x9728 1.1); W8 of
+// 5 to 8 rows .87-1.26 plain, .71-1.11 SwiGLU; W8 of 3 and 4 rows stay (plain
+// .94-1.43). By these lines 3570 measured calls take 1.004 times the better path's
+// time (geometric mean), and one is more than 3% slower than the other path; with
+// every call of up to 64 rows and a line on code bytes beyond they took 1.05
+// times, 514 of them slower, up to 2.9 times (512x19456 W8 of 129 rows).
+static bool skinny_gains(int rows, const Geometry& g, bool swiglu, bool gemv, const SkinnyPlan& p) {
+    const int K = g.K_pad, cus = device_cus();
+    const bool w4 = g.bits == 4;
+    const int groups = (rows + 16 * p.row_tiles - 1) / (16 * p.row_tiles);
+    const long long blocks = (long long)p.blocks_n * groups;
+    const long long per_cu = (blocks + cus - 1) / cus;
+    if (gemv) {
+        const bool full = 5 * blocks >= 3 * per_cu * cus;  // (the last round's CUs mostly have a block)
+        if (rows <= 2) return false;
+        if (w4) return rows > 4 || swiglu || K < 3072 || full;
+        if (rows <= 4) return false;
+        if (swiglu) return per_cu == 1 || K >= (per_cu == 2 ? 1024 : 2560);
+        return K >= 2048 && K <= 4096 && (per_cu == 1 || (K >= 2560 && full));
+    }
+    if (swiglu) {
+        if (p.row_tiles == 8) return per_cu <= (w4 ? 2 : 1) && K < 8192;
+        return per_cu <= 3 || (per_cu == 4 && (w4 || (p.row_tiles == 1 && K <= 4096)));
+    }
+    switch (p.row_tiles) {
+        case 1: return w4 ? per_cu <= 3 || K >= 2560 : per_cu == 1 || (per_cu == 2 && K >= 1024);
+        case 2: return w4 ? per_cu <= 2 || (per_cu == 3 && K >= 1536) : per_cu == 1 || (per_cu == 2 && K >= 2560);
+        case 4: return w4 ? per_cu == 1 || (per_cu == 2 && K >= 1536 && K < 8192) : per_cu == 1 && K < 8192;
+        default: return per_cu == 1 && K < 8192 && (w4 || K >= 1536 || (p.col_tiles == 1 && g.N_pad <= 2560));
+    }
+}
 
+// Whether a call of `rows` rows runs on skinny_kernel, and how: one column tile
+// per block while the blocks fit one per CU, else two (o of 16 rows W4 one 7.5,
+// two 8.1 us; qkv 7.8 and 7.5, of 128 rows 14.5 and 12.2). HM_SKINNY: 0 never, 1
+// always up to SKINNY_MAX_ROWS rows. A forced GEMM tile or split
+// (HM_GEMM_VARIANT, HM_SPLITS) keeps the tiled GEMM, as does HM_FORCE_GEMM for
+// its rows unless HM_SKINNY is 1.
 static bool plan_skinny(int rows, const Geometry& g, int epi, bool gemv, SkinnyPlan& p) {
     const int forced = switch_value(SW_SKINNY);
     if (forced == 0 || rows > SKINNY_MAX_ROWS || switch_value(SW_GEMM_VARIANT) >= 0 || switch_value(SW_SPLITS) > 0)
         return false;
     if (forced < 0 && rows <= 8 && switch_value(SW_FORCE_GEMM) != 0) return false;
-    const int cus = device_cus();
     p.row_tiles = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 64 ? 4 : 8;
     const int groups = (rows + 16 * p.row_tiles - 1) / (16 * p.row_tiles);
-    p.col_tiles = epi != EPI_PLAIN || g.N_pad / 16 * groups > cus ? 2 : 1;
+    p.col_tiles = epi != EPI_PLAIN || g.N_pad / 16 * groups > device_cus() ? 2 : 1;
     // (SwiGLU: a block per pair of a gate and an up tile and none for padding
     // columns, as every block's row maxima are read; N is a multiple of 64)
     p.blocks_n = epi != EPI_PLAIN ? g.N / 32 : g.N_pad / (16 * p.col_tiles);
-    if (forced > 0) return true;
-    if (gemv && (rows <= 2 || (rows <= 4 && g.bits == 8))) return false;
-    if (rows <= 64) return true;
-    const size_t per_cu = ((size_t)p.blocks_n * groups + cus - 1) / cus;
-    return per_cu * 16 * p.row_tiles * g.K_pad <= skinny_code_bytes;
+    return forced > 0 || skinny_gains(rows, g, epi != EPI_PLAIN, gemv, p);
 }
 
 // --- workspaces -------------------------------------------------------------

@@ -34,9 +34,9 @@ namespace hm {
 // At 16 rows what is left is the two launches (about 2.3 us each) and the
 // weight stream (gate_up's 25 MB at 3.2 TB/s with its launch); from 64 rows on
 // it is the codes: a block reads 16 RT rows of all of K, at 35 bytes per clock
-// and CU, so few-row calls of up to skinny_code_bytes (hip_matmul.hip) per CU
-// come here and the rest stays with the tiled GEMM, which stages them in LDS
-// for 128 columns. Row maxima leave as one partial per row and block: met by
+// and CU, so calls come here where few blocks a CU read them (skinny_gains,
+// hip_matmul.hip) and the rest stays with the tiled GEMM, which stages them in
+// LDS for 128 columns. Row maxima leave as one partial per row and block: met by
 // atomics on the rows' few cache lines, they took gate_up of 16 rows from 12.0
 // to 15.8 us and of 64 rows from 16.5 to 23.4.
 //

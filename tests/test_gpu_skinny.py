@@ -155,3 +155,41 @@ def test_forced_gemm_is_the_tiled_one(ctx, bits, rows):
             torch.cuda.synchronize()
         assert [s["name"].startswith(kernel) for s in p.stats if s["kind"] < 2] == [True], p.stats
         assert np.array_equal(y.cpu().numpy(), oracle.linear(codes, scales, x))
+
+
+@pytest.mark.parametrize("k,n,bits,rows,swiglu,kernel", [
+    # blocks of up to 16, 32, 64 and 256 rows at the last number a CU and past it
+    (512, 24576, 4, 16, False, "skinny"), (512, 24832, 4, 16, False, "gemm"), (512, 8448, 8, 16, False, "gemm"),
+    (1024, 16384, 8, 16, False, "skinny"), (512, 16384, 4, 32, False, "skinny"), (1024, 24576, 4, 32, False, "gemm"),
+    (512, 8192, 8, 32, False, "skinny"), (512, 16384, 8, 32, False, "gemm"), (512, 8192, 4, 64, False, "skinny"),
+    (512, 16384, 4, 64, False, "gemm"), (1536, 8448, 4, 64, False, "skinny"), (512, 8448, 8, 48, False, "gemm"),
+    (512, 8192, 4, 128, False, "skinny"), (512, 16384, 4, 128, False, "gemm"), (512, 8192, 8, 128, False, "gemm"),
+    (512, 2560, 8, 128, False, "skinny"), (512, 2560, 8, 256, False, "gemm"), (1536, 8192, 8, 128, False, "skinny"),
+    (512, 8192, 8, 128, True, "skinny"), (512, 16384, 8, 128, True, "gemm"), (512, 16384, 4, 128, True, "skinny"),
+    (512, 24576, 8, 64, True, "skinny"), (512, 32768, 8, 64, True, "gemm"), (512, 33024, 4, 20, True, "gemm"),
+    # long K
+    (8192, 512, 4, 64, False, "skinny"), (8192, 512, 8, 64, False, "gemm"), (8192, 512, 4, 65, False, "gemm"),
+    # against the GEMV
+    (3072, 2304, 4, 4, False, "gemv"), (3072, 2560, 4, 4, False, "skinny"), (2048, 512, 4, 3, False, "skinny"),
+    (1536, 512, 8, 8, False, "gemv"), (2048, 512, 8, 8, False, "skinny"), (512, 512, 8, 5, True, "skinny"),
+    (512, 8448, 8, 5, True, "gemv"), (2048, 512, 8, 4, False, "gemv"),
+])
+def test_dispatch_lines(ctx, k, n, bits, rows, swiglu, kernel):
+    """Which kernel a call takes on either side of each line of the rule (256
+    CUs), and that the other path gives the same bits there."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    lo, hi = (-8, 8) if bits == 4 else (-127, 128)
+    w = ctx.weights(bits, torch.randint(lo, hi, (k, n), generator=g, device="cuda", dtype=torch.int8),
+                    torch.rand(n, generator=g, device="cuda") * 0.009 + 0.001)
+    x = torch.randn(rows, k, generator=g, device="cuda")
+    ws = ctx.workspace(bits, rows, k, n, cached=False)
+    outs = []
+    for skinny in (-1, 0 if kernel == "skinny" else 1):
+        outs.append(torch.empty(rows, n // 2 if swiglu else n, device="cuda"))
+        with D.plan_switch("HM_SKINNY", skinny), D.KernelProfile(16) as p:
+            D.linear(ctx, w, x, outs[-1], rows, swiglu=swiglu, ws=ws)
+            torch.cuda.synchronize()
+        names = [s["name"] for s in p.stats if s["kind"] < 2]
+        assert len(names) == 1 and names[0].startswith(kernel + "<") == (skinny == -1), (names, skinny)
+    assert torch.equal(*outs)
