@@ -18,13 +18,19 @@ constexpr uint32_t MAGIC_MOE_WS = 0x534d4841u;
 constexpr uint32_t BLOB_MAGIC = 0x31584d48u;  // "HMX1"
 constexpr int MOE_BM = 64, MOE_BN = 128;
 // The streamed grouped path (moe_stream.hpp) is taken up to this many slots per
-// expert of the bank: 16-row tiles up to the first, 48-row tiles up to the
-// second. hidden 2048, 128 experts, top 8, intermediate 768, W8 down, us per
-// call, tiled GEMM / 16-row / 48-row tiles: 25 tokens 95 / 65 / 72, 128 (8 slots
-// per expert) 113 / 91 / 98, 256 (16) 121 / 130 / 98, 512 (32) 138 / 214 / 119,
-// 640 (40) 144 / - / 138, 768 (48) 149 / - / 169, where runs past 48 slots make
-// a second pass over their weights.
-constexpr int STREAM_SLOTS_16 = 10, STREAM_SLOTS_48 = 40;
+// expert of the bank: 16-row tiles up to the first, 48-row tiles up to the last.
+// hidden 2048, 128 experts, top 8, intermediate 768, W8 down, us per call, tiled
+// GEMM / 16-row / 48-row tiles: 25 tokens 95 / 65 / 72, 128 (8 slots per expert)
+// 113 / 91 / 98, 256 (16) 121 / 130 / 98, 512 (32) 138 / 214 / 119, 640 (40) 144 /
+// - / 138, 768 (48) 149 / - / 169, where runs past 48 slots make a second pass over
+// their weights. Over hidden 1024 to 2048, intermediate 256 to 1024, 32 to 128
+// experts, W4 and W8 down, distinct banks from HBM, time over the tiled GEMM's: 6 to
+// 10 slots .64-.89, 12 to 24 .71-.92, 28 and 32 .74-.97, 36 .80-1.00, 40 .83-1.07. (A
+// bank that stays in the caches between calls: up to 1.0 at 14, 1.1 at 28, 1.16 at 32.)
+// Where neither product's K fits the register window (hidden 2880 to 4096,
+// intermediate 1536 to 2880): 4 slots .84-.97, 6 .87-1.00, 8 .94-1.04, 10 1.06-1.07;
+// where one does, up to 10 .74-.99.
+constexpr int STREAM_SLOTS_16 = 10, STREAM_SLOTS_16_RELOADED = 6, STREAM_SLOTS_48 = 36;
 // Longest intermediate whose codes a block of the 16-row tiles quantizes itself
 // (32 KB of LDS); longer ones are quantized by a launch.
 constexpr int STREAM_AQ_K = 2048;
@@ -353,9 +359,9 @@ static void launch_slot_gemv(const GemvParams& V, int slots, hipStream_t s) {
 // reloaded window they lose (hidden 4096, intermediate 1536, 64 experts, 256
 // tokens: 249 us against 211 tiled; 16-row tiles at 30 tokens 171 against 183).
 static int stream_tile(int slots, const MoeBank* b) {
-    if (slots <= STREAM_SLOTS_16 * b->experts) return 16;
-    const bool held = stream_holds(4, b->ggu.K_pad) && stream_holds(b->dn_bits, b->gdn.K_pad);
-    return held && slots <= STREAM_SLOTS_48 * b->experts ? 48 : 0;
+    const bool gu = stream_holds(4, b->ggu.K_pad), dn = stream_holds(b->dn_bits, b->gdn.K_pad);
+    if (slots <= (gu || dn ? STREAM_SLOTS_16 : STREAM_SLOTS_16_RELOADED) * b->experts) return 16;
+    return gu && dn && slots <= STREAM_SLOTS_48 * b->experts ? 48 : 0;
 }
 
 // The streamed grouped path up to the contributions: routing and the tokens'

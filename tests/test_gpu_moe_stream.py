@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle
+from open_rknpu2_lm_infer_amd import device as D
 from open_rknpu2_lm_infer_amd import npu
 from tests import refdata as R
 from tests.test_gpu_ffn_moe import moe_bank, routed
@@ -52,3 +53,18 @@ def test_run_lengths(runs, dn_bits):
     rows = len(flat)
     w = R.rng_for(6, f"runs-w{rows}").uniform(0.1, 1.0, (rows, 1)).astype(np.float32)
     check(192, 96, len(runs), dn_bits, rows, 1, flat[:, None].copy(), w, f"runs-{rows}-{len(runs)}-{dn_bits}")
+
+
+@pytest.mark.parametrize("h,inter,experts,dn_bits,rows,stream", [
+    (64, 32, 4, 4, 72, True), (64, 32, 4, 8, 73, False),           # 36 slots per expert, both windows held
+    (2112, 64, 7, 8, 35, True), (2112, 64, 7, 8, 36, False),       # 10, gate/up reloaded
+    (2112, 1056, 11, 8, 33, True), (2112, 1056, 11, 8, 34, False)])  # 6, both reloaded
+def test_dispatch_lines(h, inter, experts, dn_bits, rows, stream):
+    """The streamed kernels up to their number of slots per expert, the tiled
+    grouped GEMM past it."""
+    tag = f"msd-{h}-{inter}-{rows}"
+    ids, w = routed(rows, experts, 2, tag)
+    with D.KernelProfile(64) as p:
+        check(h, inter, experts, dn_bits, rows, 2, ids, w, tag)
+    names = {s["name"] for s in p.stats if s["kind"] == 3}
+    assert names == ({"moe_stream<gate_up>", "moe_stream<down>"} if stream else {"moe_gemm<gate_up>", "moe_gemm<down>"})
