@@ -45,20 +45,22 @@ def test_device_linear_matches_oracle_f32_and_f16(ctx, bits, rows):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("rows", [3, 4])
 def test_four_row_gemv_quantized_in_blocks(ctx, bits, rows):
-    """HM_GEMV_PREQ=0: the 4-row GEMV quantizes its rows inside every block
-    instead of after a quantization launch; plain and SwiGLU outputs, f32 and
-    f16 activations, identical to the oracle."""
+    """HM_GEMV_PREQ=0: the 4-row GEMV (HM_SKINNY=0 keeps W4 on it) quantizes its
+    rows inside every block instead of after a quantization launch; plain and
+    SwiGLU outputs, f32 and f16 activations, identical to the oracle."""
     k, n = 768, 768
     codes, scales = R.weights(5, f"dlq{bits}", bits, k, n)
     w = ctx.weights(bits, dev(codes), dev(scales))
     x = R.activations(5, f"dlQ-x{rows}", rows, k)
-    with D.plan_switch("HM_GEMV_PREQ", 0):
+    with D.plan_switch("HM_GEMV_PREQ", 0), D.plan_switch("HM_SKINNY", 0):
         for xin in (dev(x), dev(x).half()):
             y = torch.empty(rows, n, dtype=torch.float32, device="cuda")
-            D.linear(ctx, w, xin, y, rows)
             m = torch.empty(rows, n // 2, dtype=torch.float32, device="cuda")
-            D.linear(ctx, w, xin, m, rows, swiglu=True)
-            torch.cuda.synchronize()
+            with D.KernelProfile(16) as p:
+                D.linear(ctx, w, xin, y, rows)
+                D.linear(ctx, w, xin, m, rows, swiglu=True)
+                torch.cuda.synchronize()
+            assert all(s["name"].startswith("gemv<mr=4") for s in p.stats) and len(p.stats) == 2, p.stats
             assert np.array_equal(y.cpu().numpy(), oracle.linear(codes, scales, x))
             assert np.array_equal(m.cpu().numpy(), oracle.linear_swiglu(codes, scales, x))
 
@@ -67,8 +69,9 @@ def test_four_row_gemv_quantized_in_blocks(ctx, bits, rows):
 @pytest.mark.parametrize("k", [640, 768, 2560, 9728])
 def test_gemv_matrix_core_dots(ctx, bits, k):
     """2 to 8 rows: the GEMV's dot products on the matrix cores (K_pad a
-    multiple of 128 for W8, 256 for W4; W4 at K = 640 takes the GEMM), rows
-    quantized in the block or beforehand (HM_GEMV_PREQ), fp16 and f32 rows,
+    multiple of 128 for W8, 256 for W4; W4 at K = 640 takes the GEMM; HM_SKINNY=0
+    keeps 3 to 8 rows here), rows quantized in the block or beforehand
+    (HM_GEMV_PREQ), fp16 and f32 rows,
     plain and SwiGLU, the 512-thread two-window blocks at K = 9728: identical
     to the oracle."""
     n = 256
@@ -82,7 +85,7 @@ def test_gemv_matrix_core_dots(ctx, bits, k):
         for preq in (1, 0):
             for xin in (dev(x), dev(x).half()):
                 print(f"W{bits} K={k} rows={rows} preq={preq} {xin.dtype}", flush=True)
-                with D.plan_switch("HM_GEMV_PREQ", preq):
+                with D.plan_switch("HM_GEMV_PREQ", preq), D.plan_switch("HM_SKINNY", 0):
                     y = torch.empty(rows, n, dtype=torch.float32, device="cuda")
                     D.linear(ctx, w, xin, y, rows)
                     m = torch.empty(rows, n // 2, dtype=torch.float32, device="cuda")
@@ -297,7 +300,8 @@ def _gemv_split_k_down(ctx, splits):
 @pytest.mark.parametrize("bits", [4, 8])
 def test_long_k_split_plan_matches_oracle(ctx, bits):
     """Few tiles over a long K: the plan splits K into pieces (partials, then a
-    summing epilogue launch); results equal the oracle's."""
+    summing epilogue launch; HM_SKINNY=0 keeps W4 of 64 rows on it); results equal
+    the oracle's."""
     import ctypes
     from open_rknpu2_lm_infer_amd import _ffi as F
     rows, k, n = 64, 8192, 512
@@ -308,9 +312,10 @@ def test_long_k_split_plan_matches_oracle(ctx, bits):
     w = ctx.weights(bits, dev(codes), dev(scales))
     x = R.activations(5, "dlK-x", rows, k)
     y = torch.empty(rows, n, dtype=torch.float16, device="cuda")
-    D.linear(ctx, w, dev(x).half(), y, rows)
     m = torch.empty(rows, n // 2, dtype=torch.float32, device="cuda")
-    D.linear(ctx, w, dev(x), m, rows, swiglu=True)
+    with D.plan_switch("HM_SKINNY", 0):
+        D.linear(ctx, w, dev(x).half(), y, rows)
+        D.linear(ctx, w, dev(x), m, rows, swiglu=True)
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy(), oracle.linear(codes, scales, x).astype(np.float16))
     assert np.array_equal(m.cpu().numpy(), oracle.linear_swiglu(codes, scales, x))
