@@ -60,34 +60,26 @@ struct AttnParams {
     float max_unit;   // the partials' maxima in powers of 2: 1 (base 2) or log2(e) (natural)
 };
 
-// max / sum over the N consecutive lanes (N = 16 or 64) that share a query row
-template <int N>
-__device__ __forceinline__ float group_max(float v) {
+// max / sum over a wave
+__device__ __forceinline__ float lanes_max(float v) {
     v = fmaxf(v, dpp_move<DPP_QUAD_XOR1>(v));
     v = fmaxf(v, dpp_move<DPP_QUAD_XOR2>(v));
     v = fmaxf(v, dpp_move<DPP_ROW_HALF_MIRROR>(v));
     v = fmaxf(v, dpp_move<DPP_ROW_MIRROR>(v));
-    if constexpr (N == 64) {
-        v = fmaxf(v, dpp_move<DPP_ROW_BCAST15, 0xa>(v));
-        v = fmaxf(v, dpp_move<DPP_ROW_BCAST31, 0xc>(v));
-        v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-    }
-    return v;
+    v = fmaxf(v, dpp_move<DPP_ROW_BCAST15, 0xa>(v));
+    v = fmaxf(v, dpp_move<DPP_ROW_BCAST31, 0xc>(v));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
-template <int N>
-__device__ __forceinline__ float group_sum(float v) {
+__device__ __forceinline__ float lanes_sum(float v) {
     v = v + dpp_move<DPP_QUAD_XOR1>(v);
     v = v + dpp_move<DPP_QUAD_XOR2>(v);
     v = v + dpp_move<DPP_ROW_HALF_MIRROR>(v);
     v = v + dpp_move<DPP_ROW_MIRROR>(v);
-    if constexpr (N == 64) {
-        v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_ROW_BCAST15,
-                                                                      0xa, 0xf, false));
-        v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_ROW_BCAST31,
-                                                                      0xc, 0xf, false));
-        v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-    }
-    return v;
+    v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_ROW_BCAST15, 0xa,
+                                                                  0xf, false));
+    v = v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), DPP_ROW_BCAST31, 0xc,
+                                                                  0xf, false));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
 // An output that came out NaN, of query row qrow (within its head) of KV head g
@@ -111,36 +103,30 @@ __device__ __forceinline__ float nan_output(const AttnParams& P, int g, int qrow
     return nan || up == down ? NAN : up ? INFINITY : -INFINITY;
 }
 
-// Block: 256 threads; RT query rows (4: 64 threads per row), head_dim 256.
-// Thread (row, sub) scores key sub of each tile and owns output dims
-// [sub*DPT, sub*DPT + DPT) of its row. K/V tiles of 32 keys go through LDS;
-// the next tile's loads are in flight (registers) while the current tile is
-// computed. Left for at most 4 rows over few keys, where it is launch and
+// At most 4 rows of head_dim 256 over few keys. Block: 4 query rows, a wave
+// each. Lane sub scores key sub of each tile of 32 and owns output dims 4 sub..+3
+// of its row. K/V tiles go through LDS; the next tile's loads are in flight
+// (registers) while the current tile is computed. What is left here is launch and
 // latency: one row of 4-head groups over 1000 keys of 8 KV heads 8.7 us, on
-// attn_tile_kernel 9.2; over 300 7.2 and 8.3. Scores are
-// v_dot2_f32_f16 sums over the fp16 q and k pairs (exact products, f32
-// accumulation) times the scale; p * v folds the fp16 conversion into the
-// multiply-add.
-template <int D, int RT>
+// attn_tile_kernel 9.2; over 300 7.2 and 8.3. Scores are v_dot2_f32_f16 sums over
+// the fp16 q and k pairs (exact products, f32 accumulation) times the scale; p * v
+// folds the fp16 conversion into the multiply-add.
 __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    constexpr int KT = 32;                           // keys per tile
-    constexpr int RPT = 256 / RT;                    // threads per row
-    constexpr int SPT = KT >= RPT ? KT / RPT : 1;    // scores per thread per tile
-    constexpr int DPT = D / RPT;                     // output dims per thread
-    constexpr int KP = D + 8;                        // LDS row pitch of a K/V tile (halves)
-    constexpr int PER = (KT * (D / 8) + 255) / 256;  // 16-byte K (and V) pieces per thread per tile
-    constexpr int QPT = RT * D / 256;                // q halves per thread (2..16)
-    static_assert(DPT >= 1 && D % RPT == 0 && D % 8 == 0 && QPT % 2 == 0,
-                  "head_dim must split over the threads");
-    constexpr int QW = QPT / 2;  // q words per thread
+    constexpr int D = 256, RT = 4;
+    constexpr int KT = 32;                   // keys per tile
+    constexpr int DPT = D / 64;              // output dims per lane
+    constexpr int KP = D + 8;                // LDS row pitch of a K/V tile (halves)
+    constexpr int PER = KT * (D / 8) / 256;  // 16-byte K (and V) pieces per thread per tile
+    constexpr int QPT = RT * D / 256;        // q halves per thread
+    constexpr int QW = QPT / 2;              // q words per thread
     __shared__ __attribute__((aligned(16))) __half qs[RT][D];
     __shared__ __attribute__((aligned(16))) __half ks[KT][KP];
     __shared__ __attribute__((aligned(16))) __half vs[KT][KP];
     __shared__ float ps[RT][KT];
     const int split = blockIdx.x, rt = blockIdx.y, g = blockIdx.z;
     const int G = P.qh / P.kh, R = G * P.m;
-    const int tid = threadIdx.x, row = tid / RPT, sub = tid % RPT;
+    const int tid = threadIdx.x, row = tid / 64, sub = tid % 64;
     const int rr = rt * RT + row;
     const bool row_ok = rr < R;
     const int gi = row_ok ? rr / P.m : 0, qr = row_ok ? rr % P.m : 0;
@@ -162,7 +148,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int i = tid + 256 * t, j = i / (D / 8), c = i % (D / 8), key = kb + j;
-            const bool ok = i < KT * (D / 8) && key < k1;
+            const bool ok = key < k1;
             const size_t off = ok ? (size_t)key * D + c * 8 : 0;  // (masked: a valid row, zeroed at the store)
             kr[t] = *reinterpret_cast<const v4u*>(kbase + off);
             vr[t] = *reinterpret_cast<const v4u*>(vbase + off);
@@ -172,11 +158,9 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int i = tid + 256 * t, j = i / (D / 8), c = i % (D / 8), key = kb + j;
-            if (i < KT * (D / 8)) {
-                const bool ok = key < k1;
-                *reinterpret_cast<v4u*>(&ks[j][c * 8]) = ok ? kr[t] : v4u{0u, 0u, 0u, 0u};
-                *reinterpret_cast<v4u*>(&vs[j][c * 8]) = ok ? vr[t] : v4u{0u, 0u, 0u, 0u};
-            }
+            const bool ok = key < k1;
+            *reinterpret_cast<v4u*>(&ks[j][c * 8]) = ok ? kr[t] : v4u{0u, 0u, 0u, 0u};
+            *reinterpret_cast<v4u*>(&vs[j][c * 8]) = ok ? vr[t] : v4u{0u, 0u, 0u, 0u};
         }
     };
     if (k0 < k1) issue(k0);
@@ -191,41 +175,27 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnParams P) {
         store(kb);
         __syncthreads();
         if (kb + KT < k1) issue(kb + KT);  // next tile in flight during this one
-        float s[SPT];
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < SPT; ++i) {
-            const int j = sub + RPT * i;
-            float a = 0.0f;
-            if (j < KT) {
+        float a = 0.0f;
+        if (sub < KT) {
 #pragma unroll 4
-                for (int c = 0; c < D; c += 8) {
-                    const v4u kw = *reinterpret_cast<const v4u*>(&ks[j][c]);
-                    const v4u qw = *reinterpret_cast<const v4u*>(&qs[row][c]);
+            for (int c = 0; c < D; c += 8) {
+                const v4u kw = *reinterpret_cast<const v4u*>(&ks[sub][c]);
+                const v4u qw = *reinterpret_cast<const v4u*>(&qs[row][c]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const unsigned qu = qw[e], ku = kw[e];  // (copied out before the bit casts)
-                        a = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, qu), __builtin_bit_cast(h2, ku), a, false);
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    const unsigned qu = qw[e], ku = kw[e];  // (copied out before the bit casts)
+                    a = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, qu), __builtin_bit_cast(h2, ku), a, false);
                 }
             }
-            const int key = kb + j;
-            s[i] = (row_ok && j < KT && key < klimit && key < k1) ? a * P.scale : -INFINITY;
-            tmax = fmaxf(tmax, s[i]);
         }
-        tmax = group_max<RPT>(tmax);
-        const float mnew = fmaxf(mrun, tmax);
+        const int key = kb + sub;
+        const float s = (row_ok && sub < KT && key < klimit && key < k1) ? a * P.scale : -INFINITY;
+        const float mnew = fmaxf(mrun, lanes_max(s));
         // (a row with no visible key yet keeps max -inf, sum 0, scale 1)
         const float alpha = (mnew == -INFINITY) ? 1.0f : __expf(mrun - mnew);
-        float psum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < SPT; ++i) {
-            const float p = (s[i] == -INFINITY) ? 0.0f : __expf(s[i] - mnew);
-            if (sub + RPT * i < KT) ps[row][sub + RPT * i] = p;
-            psum += p;
-        }
-        psum = group_sum<RPT>(psum);
-        lrun = lrun * alpha + psum;
+        const float p = (s == -INFINITY) ? 0.0f : __expf(s - mnew);
+        if (sub < KT) ps[row][sub] = p;
+        lrun = lrun * alpha + lanes_sum(p);
         mrun = mnew;
 #pragma unroll
         for (int e = 0; e < DPT; ++e) acc[e] *= alpha;
@@ -576,8 +546,8 @@ __global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnPar
 //   head_dim 64,  16 / 8, 1 row x 16000                        14.4 ->  9.7
 // At few rows it is launches and one or two memory round trips; at many, the
 // LDS reads of a fragment per 16 rows, the exponentials and the products,
-// which the two waves of a SIMD overlap only in part (head_dim 256: 0.7 us per
-// 64 keys of a 64-row block). RW = 2 (a fragment read serves 32 rows) and
+// which the two waves of a SIMD overlap only in part (head_dim 256: about 2 us
+// per 64 keys of a 64-row block, the 138 us above being 64 such stages). RW = 2 (a fragment read serves 32 rows) and
 // 4-wave blocks of 64 or 128 rows were slower at every size tried.
 constexpr float ATTN_SHIFT = 7.0f;
 
@@ -857,13 +827,13 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams P) {
     }
     const float m = tid < S ? p0[tid * STRIDE] : -INFINITY;
     const float l = tid < S ? p0[tid * STRIDE + 1] : 0.0f;
-    float mx = group_max<64>(m);
+    float mx = lanes_max(m);
     if (lane == 0) red[0][wave] = mx;
     __syncthreads();
     mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     const float w = (m == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * P.max_unit);
     w_s[tid] = w;
-    const float den = group_sum<64>(w * l);
+    const float den = lanes_sum(w * l);
     if (lane == 0) red[1][wave] = den;
     __syncthreads();
     float num[ND];
@@ -931,9 +901,9 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(AttnParams P) {
     }
     const float m = lane < S ? p0[lane * STRIDE] : -INFINITY;
     const float l = lane < S ? p0[lane * STRIDE + 1] : 0.0f;
-    const float mx = group_max<64>(m);
+    const float mx = lanes_max(m);
     const float w = (m == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * P.max_unit);
-    const float den = group_sum<64>(w * l);
+    const float den = lanes_sum(w * l);
     float num[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) num[d] = 0.0f;
@@ -1250,10 +1220,11 @@ struct AttnPlan {
 // - head_dim 64 and 128, R < 16: attn_tile_kernel of 32 rows, weights in 32
 //   bits, 4 waves so that two blocks share a CU (one row of 4-head groups over
 //   3968 keys 8.4; blocks of 16 rows 8.5, of 64 and 8 waves 9.3).
-// - R >= 16: attn_tile_kernel of 64 rows, fp16 weights; 128 rows or more
+// - R >= 16: attn_tile_kernel of 64 rows, fp16 weights; more than 64 rows
 //   attn_wide_kernel once a CU's share of the work passes 640 keys of a
 //   64-row tile (8 heads: 512 rows x 2028 keys, 507 keys a CU, 20.6 wide and
-//   19.0 tiles; 512 x 4096, 1024 keys, 25.0 and 26.9).
+//   19.0 tiles; 512 x 4096, 1024 keys, 25.0 and 26.9; 96 rows, two thirds of a
+//   wide block, x 16000, 1000 keys, 23.8 and 26.3).
 // Keys: enough splits that about 512 of the 4-wave blocks run, 256 of the
 // 8-wave ones (one per CU), each split a whole number of tiles; with more than
 // one split the blocks write partials (enqueue_attention checks that the
@@ -1305,7 +1276,7 @@ template <int D>
 static void launch_attn(const AttnParams& P, const AttnPlan& pl, const dim3& grid, hipStream_t s) {
     if constexpr (D == 256) {
         if (pl.kernel == ATTN_VALU)
-            hipLaunchKernelGGL((attn_split_kernel<256, 4>), grid, dim3(256), 0, s, P);
+            hipLaunchKernelGGL(attn_split_kernel, grid, dim3(256), 0, s, P);
         else
             hipLaunchKernelGGL((attn_tile_kernel<256, 4, 2, true>), grid, dim3(512), 0, s, P);
     } else {
