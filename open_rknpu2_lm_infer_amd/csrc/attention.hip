@@ -512,10 +512,10 @@ __global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnPar
 // WK waves share a row group's keys and their partial (max, sum, accumulators)
 // meet in LDS at the end; waves whose rows or keys are all masked skip their
 // products. Operands and lane layouts are attn_wide_kernel's: S^T = K Q^T,
-// softmax in place, O^T += V^T P^T with transposing V reads. Stages go global -> registers -> one of two LDS buffers: stage
-// t + 1 is in registers while stage t is computed, then stored to the buffer
-// stage t - 1 left (every wave passed the barrier after it), one barrier per
-// stage.
+// softmax in place, O^T += V^T P^T with transposing V reads. Stages go global ->
+// registers -> one of two LDS buffers: stage t + 1 is in registers while stage t
+// is computed, then stored to the buffer stage t - 1 left (every wave passed the
+// barrier after it), one barrier per stage.
 //
 // SPLIT: the softmax weights keep f32's precision on the fp16 matrix cores as
 // a sum of two fp16 (p = ph + pl, pl = the rounded remainder: 22 bits of p),
@@ -530,8 +530,17 @@ __global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnPar
 // keys and every head_dim, each at three spreads of the scores, the error is
 // 0.59 times theirs (geometric mean; largest at normal q and k 4.6e-7, theirs
 // 1.4e-6). An infinite value leaves NaN with a remainder of 0 or below;
-// nan_output puts that right. Calls that had fp16 weights keep them (SPLIT =
-// false).
+// nan_output puts that right.
+//
+// Calls that had fp16 weights keep them (SPLIT = false). There the maximum is not
+// lazy over a wave's first two stages, 64 keys: the largest weight among them is
+// then exactly 1, as in the 64-key tiles of the 4-wave blocks these calls had.
+// With a lazy one its rounding showed: 1.13 times those blocks' error against 64
+// bits on 64 rows of 8 heads over 4000 keys, 3.9 times with 4 times wider scores.
+// Now at most the same over 78 shapes of 16 to 800 rows per KV head at normal q and k
+// (0.94 times, geometric mean), in the same time (those 64 rows with their append
+// 16.6 and 16.5 us, 512 rows over 2000 keys 20.3 and 20.4); exact to the end of
+// longer chains they take up to 5% longer.
 //
 // Measured per run with its combine, us, the kernels before -> this (one row =
 // one query row, so 4 or 8 rows per KV head):
@@ -547,8 +556,9 @@ __global__ __launch_bounds__(64 * ATTN_WIDE_WAVES) void attn_wide_kernel(AttnPar
 // At few rows it is launches and one or two memory round trips; at many, the
 // LDS reads of a fragment per 16 rows, the exponentials and the products,
 // which the two waves of a SIMD overlap only in part (head_dim 256: about 2 us
-// per 64 keys of a 64-row block, the 138 us above being 64 such stages). RW = 2 (a fragment read serves 32 rows) and
-// 4-wave blocks of 64 or 128 rows were slower at every size tried.
+// per 64 keys of a 64-row block, the 138 us above being 64 such stages). RW = 2 (a
+// fragment read serves 32 rows) and 4-wave blocks of 64 or 128 rows were slower at
+// every size tried.
 constexpr float ATTN_SHIFT = 7.0f;
 
 template <int D, int WR, int WK, bool SPLIT>
@@ -667,16 +677,18 @@ __global__ __launch_bounds__(64 * WR * WK) void attn_tile_kernel(AttnParams P) {
                         if (!(key < lim && key < k1)) sacc[cb][r] = -INFINITY;
                     }
             }
+            // (the maximum follows the scores from this rise on)
+            const float lazy = SPLIT || kb >= k0 + 2 * KT ? ATTN_LAZY : 0.0f;
             float lmax = -INFINITY;
 #pragma unroll
             for (int cb = 0; cb < 2; ++cb)
                 lmax = __builtin_elementwise_maximum(
                     __builtin_elementwise_maximum(lmax, __builtin_elementwise_maximum(sacc[cb][0], sacc[cb][1])),
                     __builtin_elementwise_maximum(sacc[cb][2], sacc[cb][3]));
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(lmax * c > mrun + (ATTN_LAZY + SHIFT)) != 0, 0)) {
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(lmax * c > mrun + (lazy + SHIFT)) != 0, 0)) {
                 const float tm = max_rows4(lmax) * c - SHIFT;
                 float alpha = 1.0f;
-                if (tm > mrun + ATTN_LAZY) {
+                if (tm > mrun + lazy) {
                     alpha = __builtin_amdgcn_exp2f(mrun - tm);  // (0 from -inf)
                     mrun = tm;
                 }

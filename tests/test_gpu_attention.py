@@ -577,3 +577,49 @@ def test_infinite_values(d, qh, kh, rows, length, where):
     finally:
         L.rk_npu_attention_f16_cache_free(cache)
         L.rk_npu_attention_f16_workspace_free(ws)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_largest_fp16_weight_is_exact(d):
+    """With fp16 weights a row's largest weight among the first 64 keys of a key
+    group is 1, so it carries no rounding, in whichever of their two stages its key
+    is. Here key 70 holds 0.4 of the weight, 127 keys the rest and the others (score
+    -24) nothing; against the maximum of the keys before it, its weight would be
+    2^6.0007, 64.031, which fp16 rounds by 4.9e-4: 0.4 * 0.6 * 4.9e-4 = 1.2e-4 of
+    the values, about 2e-4 of the output. The other weights round by 2e-4 (rms)
+    each, which over 127 of them is 127**-0.5 * 0.6 * 2e-4 = 1e-5: 5e-5 lies
+    between."""
+    L = F.lib()
+    be = npu.Backend(npu.ModelOptions(chunk=16, context=64))
+    heads, rows, length = 32, 64, 1024  # (64-row tiles, two 64-key stages a split)
+    cfg = F.rk_npu_attention_f16_config()
+    L.rk_npu_attention_f16_config_init(ctypes.byref(cfg))
+    scale = np.float32(np.log(2.0))  # (scores in powers of 2)
+    cfg.query_heads, cfg.kv_heads, cfg.head_dim, cfg.softmax_scale = heads, heads, d, float(scale)
+    cfg.max_query_rows, cfg.max_capacity, cfg.initial_capacity = rows, length, length
+    cfg.mask_mode = F.RK_NPU_ATTENTION_F16_NO_MASK
+    ws, cache = ctypes.c_void_p(), ctypes.c_void_p()
+    npu.check(L.rk_npu_attention_f16_prepare(be.domain, ctypes.byref(cfg), ctypes.byref(ws)), "prepare")
+    npu.check(L.rk_npu_attention_f16_cache_create(be.domain, ctypes.byref(cfg), ctypes.byref(cache)), "cache")
+    try:
+        g = torch.Generator(device="cuda").manual_seed(d)
+        q = torch.zeros(heads, rows, d, device="cuda").half()
+        q[:, :, :2] = 1.0
+        k = torch.zeros(heads, length, d, device="cuda").half()
+        k[:, :, 0] = -24.0
+        k[:, :128, 0] = -torch.rand(heads, 128, generator=g, device="cuda").half()
+        k[:, 0, 0] = 0.0
+        k[:, 70, 0], k[:, 70, 1] = 6.0, 0.0007
+        v = torch.randn(heads, length, d, generator=g, device="cuda").half()
+        out = torch.empty(heads, rows, d, device="cuda")
+        stream = torch.cuda.current_stream().cuda_stream
+        npu.check(L.rk_npu_hip_attention_cache_append(cache, k.data_ptr(), v.data_ptr(), length, stream), "append")
+        npu.check(L.rk_npu_hip_attention_run(ws, cache, q.data_ptr(), rows, 0, out.data_ptr(), 0, stream), "run")
+        torch.cuda.synchronize()
+        want = oracle.attention(q.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), float(scale), 0, False)
+        err = np.linalg.norm(out.cpu().numpy() - want) / np.linalg.norm(want)
+        print(f"d={d} relative error {err:.2g}", flush=True)
+        assert err < 5e-5
+    finally:
+        L.rk_npu_attention_f16_cache_free(cache)
+        L.rk_npu_attention_f16_workspace_free(ws)
