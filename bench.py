@@ -160,15 +160,15 @@ def graph_time(torch, fn, reps, check=None):
     return e0.elapsed_time(e1) / reps, ok
 
 
-# HBM bytes per launch of the dominant decode kernel (the gate_up GEMV) at
+# HBM bytes per launch of the dominant decode kernel (the gate_up product) at
 # M=1 and M=4, from two rocprofv3 counter runs of `bench.py --traffic-probe`
 # (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch, medians over 216
 # dispatches), each scaled by what the same counter reads for the run's
 # 268,435,456-byte device copy: FETCH_SIZE 131,083.5 KiB (factor 2.0),
-# WRITE_SIZE 262,144 KiB (factor 1.0). Commands and every decode GEMV's
+# WRITE_SIZE 262,144 KiB (factor 1.0). Commands and the other products'
 # figures: profiles/traffic_decode_gemv_m1_m4.txt.
-TRAFFIC_GEMV_GATE_UP = {1: int(round((12429.5 * 2.0 + 81.1 * 1.0) * 1024)),
-                        4: int(round((12466.5 * 2.0 + 304.0 * 1.0) * 1024))}
+TRAFFIC_GATE_UP = {1: int(round((12434.0 * 2.0 + 81.1 * 1.0) * 1024)),
+                   4: int(round((12446.5 * 2.0 + 152.0 * 1.0) * 1024))}
 
 
 ROOF_METHOD = "graph of 36 back-to-back launches (distinct weights), HIP events on the replay stream"
@@ -395,13 +395,14 @@ def run_decode(torch, ctx, rows, steps, warmup, want_cpu, want_roofline=True, ti
         log(f"[bench] decode M={rows}: eager {ms_eager:.3f} ms/step, graph {ms_graph:.3f} ms/step "
             f"(replay bit-exact: {ok}) -> {out['value']:.1f} GB/s; max |qkv|, |o|, |ffn| {t.magnitudes()}")
     if want_roofline:
-        # Dominant kernel: the gate_up GEMV (25 MB of W4 weights per launch).
+        # Dominant kernel: the gate_up product (25 MB of W4 weights per launch).
         passes = decode_passes(torch, ctx, t, reps or steps)
         gu = passes["gate_up"]
         out["projections"] = passes
-        out["roofline"] = roof_of("hbm", f"gemv_kernel (W4, SwiGLU epilogue) gate_up 2560x19456, M={rows}",
+        kernel = "gemv_kernel" if rows == 1 else "quant_rows_kernel + skinny_kernel"
+        out["roofline"] = roof_of("hbm", f"{kernel} (W4, SwiGLU epilogue) gate_up 2560x19456, M={rows}",
                                   gu["bytes"], gu["us"], LAYERS * (reps or steps),
-                                  traffic=TRAFFIC_GEMV_GATE_UP.get(rows))
+                                  traffic=TRAFFIC_GATE_UP.get(rows))
         # The measured ceiling of one launch of this size: a plain read of the
         # same bytes with the same loads, launched the same way.
         read_us = stream_read_us(torch, gu["bytes"])
@@ -826,7 +827,7 @@ def run_moe(torch, ctx, steps, warmup, tokens_list=(512, 1), want_cpu=True):
         else:
             res.update(value=round((routed_bytes + shared_bytes) / (ms * 1e-3) / 1e9, 1), unit="GB/s")
         parts = ("slot GEMVs W4 gate_up + W8 down, combine" if T == 1 else
-                 "route, quantization into slot order, grouped W4 gate_up + W8 down GEMMs, combine")
+                 "routing and codes, streamed W4 gate_up + W8 down products, combine")
         res["roofline"] = roof_of("hbm", f"MoE call T={T} ({parts}) + shared FFN call", routed_bytes + shared_bytes,
                                   ms * 1e3,
                                   steps * (10 if T == 1 else 1),
@@ -914,7 +915,7 @@ def run_attention(torch, ctx, steps, layers=36, length=4096, want_cpu=True):
                                   f"{layers} layers", "value": round(kv_bytes / (ms * 1e-3) / 1e9, 1),
                       "unit": "GB/s", "ms_per_step": round(ms, 4), "us_per_layer": round(us_layer, 2),
                       "graph_matches_eager": ok,
-                      "roofline": roof_of("hbm", "attention decode call (split kernel + combine), one layer",
+                      "roofline": roof_of("hbm", "attention decode call (key-split tiles + combine), one layer",
                                           kv_layer, us_layer, layers * steps,
                                           method="per layer of the step: 36 calls on distinct caches in the step, "
                                                  "faster of eager and graph replay; HIP events")}
@@ -1466,8 +1467,12 @@ def _kname(name):
     """A kernel's demangled name without the namespace and parameter list."""
     name = name[5:] if name.startswith("void ") else name
     name = name.replace("hm::", "")
-    i = name.rfind("(")
-    return name[:i] if i > 0 else name
+    depth = 0
+    for i, c in enumerate(name):
+        depth += (c == "<") - (c == ">")
+        if c == "(" and depth == 0 and i > 0 and not name.startswith("(anonymous namespace)", i):
+            return name[:i]
+    return name
 
 
 def _trace(path):
@@ -1525,8 +1530,8 @@ def _roof_passes(bench, roof):
          R["gate_up"]["us"]),
         ("decode M=1 down 9728x2560 W4 (second launch of the FFN call)",
          [(["gemv_kernel<float, 1, 4, 0,", "true>"], 327680)], lin_bytes(4, F, H, 1), "hbm", P[dn]["us"], R[dn]["us"]),
-        ("decode M=4 gate_up W4 +SwiGLU (quantization launch + GEMV)",
-         [(["quant_rows_kernel<__half, 0,"], 1024), (["gemv_kernel<float, 4, 4, 2,"], 311296)],
+        ("decode M=4 gate_up W4 +SwiGLU (quantization launch + product)",
+         [(["quant_rows_kernel<__half, 0,"], 1024), (["skinny_kernel<4, 1, 2, 2,"], 155648)],
          lin_bytes(4, H, 2 * F, 4), "hbm", _sec(bench, "decode M=4")["roofline"]["avg_us"],
          roof["decode M=4"]["roofline"]["avg_us"]),
         ("prefill M=4096 gate_up W4 +SwiGLU (quantization launch + GEMM)",
@@ -1596,10 +1601,9 @@ TRAFFIC_SPEC = [
     ("M=1 gate_up 2560x19456 +SwiGLU", ["gemv_kernel<__half, 1, 4, 2,"], 389120, lin_bytes(4, H, 2 * F, 1)),
     ("M=1 down 9728x2560 (split K, f32 middle in)", ["gemv_kernel<float, 1, 4, 0,", "true>"], 327680,
      lin_bytes(4, F, H, 1)),
-    ("M=4 qkv (rows quantized beforehand)", ["gemv_kernel<float, 4, 4, 0,"], 196608, lin_bytes(4, H, Q + 2 * KV, 4)),
-    ("M=4 o", ["gemv_kernel<float, 4, 4, 0,"], 81920, lin_bytes(4, Q, H, 4)),
-    ("M=4 gate_up +SwiGLU", ["gemv_kernel<float, 4, 4, 2,"], 311296, lin_bytes(4, H, 2 * F, 4)),
-    ("M=4 down (512-thread blocks)", ["gemv_kernel<float, 4, 4, 0,"], 163840, lin_bytes(4, F, H, 4)),
+    # (o and down of M=4 are one kernel of one grid, so their dispatches cannot be told apart)
+    ("M=4 qkv (rows quantized beforehand)", ["skinny_kernel<4, 1, 2, 0,"], 49152, lin_bytes(4, H, Q + 2 * KV, 4)),
+    ("M=4 gate_up +SwiGLU", ["skinny_kernel<4, 1, 2, 2,"], 155648, lin_bytes(4, H, 2 * F, 4)),
 ]
 
 
@@ -1620,7 +1624,7 @@ def profile_traffic(fetch_csv, write_csv):
         raise ValueError(f"calibration copy: {cal}")
     cf, cw = fe[cal[0]][0], wr[cal[0]][0]
     ff, fw = 262144.0 / cf, 262144.0 / cw
-    out = ["HBM traffic of the decode GEMVs (M=1 and M=4, W4 weights, Qwen3-4B-shaped projections), one MI355X.", "",
+    out = ["HBM traffic of the decode products (M=1 and M=4, W4 weights, Qwen3-4B-shaped projections), one MI355X.", "",
            "Commands (repository root; two counter runs of the same workload, each in its own process):",
            PROFILE_SETUP,
            "  rocprofv3 --pmc FETCH_SIZE --output-format csv -d <out_fetch> -o run -- python3 -u bench.py --traffic-probe",
@@ -1646,7 +1650,7 @@ def profile_traffic(fetch_csv, write_csv):
     out += ["", "Algorithmic bytes: weights at 4 bits + f32 column scales + fp16 activations in and out (the f32",
             "middle of the down projection and the row-max partials are not counted). A ratio near 1 means every",
             "weight byte is read from HBM once and nothing else of size is: the gap to the 8 TB/s roofline is time,",
-            "not bytes. bench.py's primary roofline carries traffic = the M=1 gate_up row (TRAFFIC_GEMV_GATE_UP)."]
+            "not bytes. bench.py's primary roofline carries traffic = the M=1 gate_up row (TRAFFIC_GATE_UP)."]
     return "\n".join(out)
 
 
@@ -1909,11 +1913,10 @@ def profile_moe(stats_csv, moe_json):
            "> moe.json",
            "  python3 bench.py --profile moe <out>/<host>/<pid>_run_kernel_stats.csv moe.json", "",
            "Workload: rk_npu_hip_moe_run at T=512 and T=1 tokens, steps of both sizes mixed in the table (eager and",
-           "graph replays). T=512: device routing (counting sort of the (token, rank) slots), the tokens'",
-           "quantization written straight into slot order (one launch, rows through the routing's slot map),",
-           "grouped gate_up GEMM + SwiGLU + row max over the ragged expert groups, middle requantization, grouped",
-           "down GEMM, combine; the shared expert as a dense FFN. T=1: slot GEMVs (slot = assignment, no routing",
-           "launch) for gate_up and down, the shared expert's GEMVs, combine.", ""]
+           "graph replays). T=512: device routing (counting sort of the (token, rank) slots) and the tokens'",
+           "codes in the same launch, streamed gate_up product + SwiGLU + row maxima over the ragged expert groups,",
+           "middle requantization, streamed down product, combine; the shared expert as a dense FFN. T=1: slot",
+           "GEMVs (slot = assignment, no routing launch) for gate_up and down, the shared expert's GEMVs, combine.", ""]
     out += _stats_table(stats_csv)
     out += ["", "bench.py --only moe in the same profiled run:"]
     for r in (res if isinstance(res, list) else [res]):
@@ -1937,7 +1940,7 @@ def profile_attention(stats_csv, attn_json, pmc1_csv, pmc2_csv):
            "  python3 bench.py --profile attention <out>/<host>/<pid>_run_kernel_stats.csv attn.json \\",
            "      <pmc1>/<host>/<pid>_run_counter_collection.csv <pmc2>/<host>/<pid>_run_counter_collection.csv", "",
            "Workload (bench.py run_attention): one rk_npu_hip_attention_run per layer cache; decode = 1 query row at",
-           "the last position (attn_split_kernel + attn_combine_kernel), prefill = 128 query rows ending at the last",
+           "the last position (attn_tile_kernel + attn_combine_kernel), prefill = 128 query rows ending at the last",
            "position, causal (attn_wide_kernel + attn_combine_rows_kernel); eager steps and graph replays both in",
            "the table.", ""]
     out += _stats_table(stats_csv)

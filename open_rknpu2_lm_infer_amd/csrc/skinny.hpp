@@ -21,9 +21,9 @@ namespace hm {
 // What it is for: the tiled GEMM walks K with one block per output tile and a
 // barrier per 64 k, so with few rows its time is K / 64 times a stage's latency
 // on the few CUs that have a tile, whatever the bytes. Here K is NWV chains per
-// column tile, on 4 to 8 times as many blocks. Measured per call, the rows'
-// quantization (3.5 us) included, distinct weights from HBM, us, tiled GEMM ->
-// this kernel:
+// column tile, on 4 to 8 times as many blocks. Measured per call in a graph, the
+// rows' quantization launch included (a kernel of 3.4 us at 16 rows, 4.1 to 4.7 at
+// 64, in a kernel trace), distinct weights from HBM, us, tiled GEMM -> this kernel:
 //                              16 rows        64 rows        128 rows
 //   o       4096x2560   W4  19.4 ->  7.5   19.1 ->  9.6   19.7 -> 13.0
 //   o       4096x2560   W8  18.6 ->  8.5   19.6 -> 11.4   20.7 -> 14.6
