@@ -177,7 +177,8 @@ def test_forced_gemm_is_the_tiled_one(ctx, bits, rows):
 def test_dispatch_lines(ctx, k, n, bits, rows, swiglu, kernel):
     """Which kernel a call takes on either side of each line of the rule (256
     CUs), and that the other path gives the same bits there."""
-    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes lie at the lines of 256 CUs")
     g = torch.Generator(device="cuda").manual_seed(k + n)
     lo, hi = (-8, 8) if bits == 4 else (-127, 128)
     w = ctx.weights(bits, torch.randint(lo, hi, (k, n), generator=g, device="cuda", dtype=torch.int8),
